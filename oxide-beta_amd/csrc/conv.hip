@@ -31,7 +31,8 @@
 //     matrix cores), as do the weight gradients (k in fixed chunks): deterministic, within
 //     1e-5 * sum|terms| of the CPU's serial sum.
 //   * Ungrouped K x K convolutions with small planes stage one image's planes and a channel
-//     tile's weights in LDS per block; the rest (and depthwise convolutions not fused with
+//     tile's weights in LDS per block; larger ones run on the matrix cores over flattened
+//     positions (conv_mfma.hip); the rest (and depthwise convolutions not fused with
 //     their BatchNorm, depthwise_bn.hip) run one output (or input, or weight-chunk) element
 //     per thread.
 #include <hip/hip_runtime.h>
@@ -41,6 +42,7 @@
 
 #include "chunk_sum.h"
 #include "common.h"
+#include "conv_mfma.h"
 
 namespace {
 
@@ -2359,6 +2361,11 @@ int tap_kernel(const ConvGeom &g) {
   return static_cast<int>(10 * g.kh + g.stride);
 }
 
+oxh::conv_mfma::Dims mfma_dims(const ConvGeom &g) {
+  return oxh::conv_mfma::Dims{g.batch, g.in_c, g.h, g.w, g.out_c, g.kh, g.stride, g.pad,
+                              g.oh, g.ow};
+}
+
 // Plans of the LDS-staged per-image kernels: `tile` channels per block (0: not applicable).
 struct LdsPlan {
   uint32_t tile = 0, tiles = 0, chunks = 1, per_chunk = 0, lds_bytes = 0;
@@ -2645,6 +2652,32 @@ MfmaWeightPlan weight_mfma_plan(const ConvGeom &g, bool bias = false) {
   p.blocks = (f.jobs + 3) / 4;
   p.lds_bytes = static_cast<uint32_t>(floats * 4);
   return p;
+}
+
+// Ungrouped square convolutions run on the matrix cores over flattened positions (conv_mfma.h)
+// where no per-image LDS kernel takes them, and where one does but the layer has over 2^27
+// products: a block per image and channel tile then restages its planes for every tile (64
+// images of 64 x 14 x 14 to 64 channels, 3 x 3: 51 against 24 us forward, 57 against 24 us input
+// gradient; 16 images, 2^26.8 products: 23 us both ways; the 128-image 7 x 7 to 96-channel
+// stride-2 layer, 2^25.8: 9 against 14 us, so smaller layers keep the per-image kernels).  A
+// stride-2 input gradient has a quarter of the blocks: twice that (14 x 14 to 128 channels: 64
+// images, 2^27.8: 35 against 42 us; 128 images: 68 against 43 us).
+constexpr uint64_t kLargeProducts = 1ull << 27;
+uint64_t products(const ConvGeom &g) {
+  return static_cast<uint64_t>(g.batch) * g.oh * g.ow * g.out_c * g.in_per_group * g.kh * g.kw;
+}
+bool large_forward(const ConvGeom &g) {
+  return g.groups == 1 && g.kh == g.kw &&
+         (products(g) > kLargeProducts ||
+          (forward_lds_plan(g).tile == 0 && forward_split_plan(g).tile == 0)) &&
+         oxh::conv_mfma::takes_forward(mfma_dims(g));
+}
+bool large_input_backward(const ConvGeom &g) {
+  return g.groups == 1 && g.kh == g.kw &&
+         (products(g) > g.stride * kLargeProducts ||
+          (input_backward_mfma_plan(g).lds_bytes == 0 &&
+           input_backward_s2_plan(g).lds_bytes == 0 && input_backward_lds_plan(g).tile == 0)) &&
+         oxh::conv_mfma::takes_input_backward(mfma_dims(g));
 }
 
 // 1x1, stride 1, no padding, one group: the convolution is a matrix product over channels.
@@ -3057,6 +3090,10 @@ oxh_status input_backward_impl(const char *name, oxh_stream stream,
     const ProductArgs x = input_product(g, gradient, weight, addend, input_gradient);
     return launch_product(name, s, x, 1, input_splits(x) != 0);
   }
+  if (large_input_backward(g)) {
+    oxh::conv_mfma::input_backward(s, mfma_dims(g), gradient, weight, addend, input_gradient);
+    return oxh::launched(name);
+  }
   const MfmaIgPlan mp = input_backward_mfma_plan(g);
   if (mp.lds_bytes > 0) {
     const dim3 mgrid(mp.tiles, g.batch), mblock(256);
@@ -3240,7 +3277,8 @@ oxh_status oxh_conv2d_output_size(const oxh_conv2d_shape *shape, uint64_t *out_h
 int oxh_conv2d_input_backward_serial(const oxh_conv2d_shape *shape) {
   ConvGeom g;
   if (make_conv_geom("oxh_conv2d_input_backward_serial", shape, g) != OXH_OK) return -1;
-  if (!pointwise(g)) return input_backward_mfma_plan(g).lds_bytes > 0 ? 0 : 1;
+  if (!pointwise(g))
+    return input_backward_mfma_plan(g).lds_bytes > 0 || large_input_backward(g) ? 0 : 1;
   return input_splits(input_product(g, nullptr, nullptr, nullptr, nullptr)) != 0 ? 0 : 1;
 }
 
@@ -3248,7 +3286,7 @@ int oxh_conv2d_forward_serial(const oxh_conv2d_shape *shape) {
   ConvGeom g;
   if (make_conv_geom("oxh_conv2d_forward_serial", shape, g) != OXH_OK) return -1;
   if (pointwise(g)) return split_kind(g.out_c, g.batch * g.h * g.w, g.in_c, 1) != 0 ? 0 : 1;
-  return forward_split_plan(g).tile > 0 ? 0 : 1;
+  return forward_split_plan(g).tile > 0 || large_forward(g) ? 0 : 1;
 }
 
 oxh_status oxh_conv2d_forward(oxh_stream stream, const oxh_conv2d_shape *shape,
@@ -3279,6 +3317,10 @@ oxh_status oxh_conv2d_forward(oxh_stream stream, const oxh_conv2d_shape *shape,
     a.K = g.in_c;
     a.k_chunk = a.K;
     return launch_product(name, s, a, 1, true);
+  }
+  if (large_forward(g)) {
+    oxh::conv_mfma::forward(s, mfma_dims(g), input, weight, bias, output);
+    return oxh::launched(name);
   }
   const MfmaForwardPlan mp = forward_mfma_plan(g);
   if (mp.lds_bytes > 0 && oxh::aligned16(input) && oxh::aligned16(weight)) {
@@ -3449,8 +3491,8 @@ oxh_status oxh_conv2d_backward(oxh_stream stream, const oxh_conv2d_shape *shape,
   }
   // a stride-2 K x K convolution whose two gradients both take the matrix-core kernels: one
   // launch (then the chunk sums and the bias launch)
-  if (!pointwise(g) && input_gradient != nullptr && oxh::aligned16(gradient) &&
-      oxh::aligned16(input)) {
+  if (!pointwise(g) && input_gradient != nullptr && !large_input_backward(g) &&
+      oxh::aligned16(gradient) && oxh::aligned16(input)) {
     const MfmaIgPlan ip = input_backward_mfma_plan(g);
     const MfmaWeightPlan wp = ip.lds_bytes > 0 ? weight_mfma_plan(g) : MfmaWeightPlan{};
     if (ip.lds_bytes > 0 && wp.lds_bytes > 0) {

@@ -1,0 +1,32 @@
+// conv_mfma.h -- ungrouped square-kernel convolutions over large planes on the matrix cores
+// (internal to the library; conv.hip chooses).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "common.h"
+
+namespace oxh {
+namespace conv_mfma {
+
+// One group, kernel k x k, the shape checks of conv.hip passed.
+struct Dims {
+  uint32_t batch, in_c, h, w, out_c, k, stride, pad, oh, ow;
+};
+
+// Whether the forward / input gradient of this convolution runs here (K x K: kernel 3 or 5, or
+// a strided or padded 1 x 1).
+bool takes_forward(const Dims &d);
+bool takes_input_backward(const Dims &d);
+
+// y[n][oc][p] = bias[oc] + sum over (ic, tap) of x * weight.
+void forward(hipStream_t s, const Dims &d, const float *x, const float *weight,
+             const float *bias, float *y);
+// dx[n][ic][p] = sum over (oc, tap) of gradient * weight (+ addend, which may be dx itself).
+void input_backward(hipStream_t s, const Dims &d, const float *gradient, const float *weight,
+                    const float *addend, float *dx);
+
+}  // namespace conv_mfma
+}  // namespace oxh

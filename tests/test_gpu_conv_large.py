@@ -1,0 +1,93 @@
+"""Convolutions over planes too large for the per-image kernels, on the matrix cores: forward,
+input gradient (with an addend) and weight / bias gradients against the oracle at the edges of
+their tiles (32 rows, 32 positions, channel pairs), within 1e-5 * sum|terms|: an fp32 sum of n
+terms in any order is off by at most n * 2^-24 * sum|terms|, and by about sqrt(n) * 2^-24 of it
+in practice, under 1e-5 for every n below 2^14."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import oxide_hip as ox
+from helpers import assert_conv_forward, assert_conv_input_gradient, host, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# batch, in, height, width, out, kernel, stride, padding
+CASES = [
+    (1, 3, 75, 73, 33, 3, 2, 1),      # a stem: one and a half channel pairs, 33 output rows
+    (2, 32, 33, 31, 32, 3, 1, 1),     # one row tile, odd planes, positions across images
+    (3, 17, 40, 29, 70, 3, 1, 1),     # an odd channel, 64 + 6 rows
+    (1, 64, 65, 66, 64, 3, 1, 1),     # whole tiles
+    (2, 40, 30, 34, 96, 3, 2, 1),
+    (2, 24, 41, 37, 40, 5, 1, 2),
+    (1, 10, 61, 43, 24, 5, 2, 2),
+    (2, 96, 32, 31, 64, 1, 2, 0),     # a strided 1 x 1: three of four inputs feed no output
+    (2, 20, 33, 33, 20, 3, 1, 0),     # no padding
+    (1, 70, 35, 20, 16, 3, 2, 0),
+    (1, 24, 35, 33, 20, 1, 1, 1),     # a padded 1 x 1
+    (20, 48, 17, 16, 66, 3, 1, 1),    # planes a per-image kernel holds, over 2^27 products
+    (60, 64, 15, 14, 144, 3, 2, 1),
+]
+
+
+def _case(case, dev):
+    n, cin, h, w, cout, k, s, pad = case
+    r = np.random.default_rng(abs(hash(case)) & 0xFFFFFFFF)
+    x = r.standard_normal((n, cin, h, w)).astype(np.float32)
+    wt = (r.standard_normal((cout, cin, k, k)) * 0.3).astype(np.float32)
+    b = r.standard_normal(cout).astype(np.float32)
+    shape = ox.conv2d_shape(n, cin, h, w, cout, k, s, pad, 1)
+    oh, ow = ox.conv2d_output_size(shape)
+    g = r.standard_normal((n, cout, oh, ow)).astype(np.float32)
+    return shape, x, wt, b, g
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_forward(module, dev, case):
+    shape, x, wt, b, g = _case(case, dev)
+    y = torch.full(g.shape, float("nan"), device=dev)
+    module.conv2d_forward(shape, to_dev(x, dev), to_dev(wt, dev), to_dev(b, dev), y)
+    assert not ox.conv2d_forward_serial(shape)
+    assert_conv_forward(host(y), x, wt, b, case[6], case[7], 1, "forward")
+
+
+@pytest.mark.parametrize("addend", ["none", "separate", "in place"])
+@pytest.mark.parametrize("case", CASES)
+def test_input_gradient(module, dev, case, addend):
+    shape, x, wt, _, g = _case(case, dev)
+    gd, wd = to_dev(g, dev), to_dev(wt, dev)
+    dx = torch.full(x.shape, float("nan"), device=dev)
+    if addend == "none":
+        module.conv2d_input_backward(shape, gd, wd, dx)
+    elif addend == "separate":
+        module.conv2d_input_backward_accumulate(shape, gd, wd, to_dev(x, dev), dx)
+    else:
+        dx = to_dev(x, dev)
+        module.conv2d_input_backward_accumulate(shape, gd, wd, dx, dx)
+    assert not ox.conv2d_input_backward_serial(shape)
+    assert_conv_input_gradient(host(dx), g, wt, case[6], case[7], 1, x.shape,
+                               None if addend == "none" else x, "input gradient")
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("case", [(2, 33, 34, 31, 40, 3, 1, 1), (1, 30, 40, 44, 66, 3, 2, 1)])
+def test_weights_that_are_not_finite(module, dev, case, value):
+    """An infinite or NaN weight reaches the outputs whose tap lies inside the input, and no
+    other: taps outside are skipped, as the CPU path skips them."""
+    shape, x, wt, b, g = _case(case, dev)
+    wt[3, 5, 0, 0] = value
+    y = torch.empty(g.shape, device=dev)
+    dx = torch.empty(x.shape, device=dev)
+    module.conv2d_forward(shape, to_dev(x, dev), to_dev(wt, dev), to_dev(b, dev), y)
+    module.conv2d_input_backward(shape, to_dev(g, dev), to_dev(wt, dev), dx)
+    ref_y = oracle.conv2d_forward(x, wt, b, case[6], case[7], 1)
+    ref_dx = oracle.conv2d_backward(g, x, wt, case[6], case[7], 1)[0]
+    for got, ref in ((host(y), ref_y), (host(dx), ref_dx)):
+        fine = np.isfinite(ref)
+        assert 0 < fine.sum() < ref.size
+        assert np.array_equal(fine, np.isfinite(got))
+        np.testing.assert_allclose(got[fine], ref[fine], rtol=1e-4, atol=1e-4)
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
