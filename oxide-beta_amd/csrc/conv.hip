@@ -2366,6 +2366,11 @@ oxh::conv_mfma::Dims mfma_dims(const ConvGeom &g) {
                               g.oh, g.ow};
 }
 
+oxh::conv_mfma::WeightDims mfma_weight_dims(const ConvGeom &g) {
+  return oxh::conv_mfma::WeightDims{g.batch, g.in_c, g.h, g.w, g.out_c, g.kh, g.kw, g.stride,
+                                    g.pad, g.oh, g.ow};
+}
+
 // Plans of the LDS-staged per-image kernels: `tile` channels per block (0: not applicable).
 struct LdsPlan {
   uint32_t tile = 0, tiles = 0, chunks = 1, per_chunk = 0, lds_bytes = 0;
@@ -2870,27 +2875,45 @@ bool depthwise_single_pass(const ConvGeom &g) {
          (g.kh == 3 || g.kh == 5) && g.out_c <= 65535 * 16;
 }
 
+// Ungrouped weight gradients the per-image matrix-core kernel (weight_mfma_plan) does not take run
+// on the matrix cores over groups of output rows (conv_weight_mfma.hip), but for short serial
+// sums: planes of at most 64 positions with an LDS plan (33 images of 5 x 7 x 7 to 9 channels:
+// 11.9 against 13.4 us; 64 images of 16 x 20 x 20: 61 against 21 us), and layers under 2^22
+// products whose generic chunks have at most 64 positions (2 images of 61 x 7 x 7 to 43: 11.7
+// against 12.4 us; 3 images of 128 x 5 x 5 to 128, 2^23.2: 14.3 against 12.8 us).  Returns the
+// partial sums it leaves, 0 where it does not run.
+uint32_t large_weight_partials(const ConvGeom &g) {
+  if (g.groups != 1) return 0;
+  const uint64_t oplane = static_cast<uint64_t>(g.oh) * g.ow;
+  if (weight_lds_plan(g).tile > 0) {
+    if (oplane <= 64) return 0;
+  } else {
+    const uint64_t chunks = weight_chunks(g);
+    if (oplane * ((g.batch + chunks - 1) / chunks) <= 64 && products(g) < (1ull << 22)) return 0;
+  }
+  return oxh::conv_mfma::weight_partials(mfma_weight_dims(g));
+}
+
 uint64_t weight_partial_bytes(const ConvGeom &g) {
   if (depthwise_single_pass(g)) return 0;
-  // the matrix-core kernel's chunks, or the LDS kernel's with room for the bias sums of a
-  // parameter-only oxh_conv2d_backward after each chunk's weights, or (operands the matrix-core
-  // kernel does not take) the generic kernel's
+  // the per-image matrix-core kernel's chunks or, where it does not take the shape or the operands'
+  // alignment, the larger of those and the partial sums of the kernel that then runs (the LDS
+  // kernel's with room for the bias sums of a parameter-only oxh_conv2d_backward after each
+  // chunk's weights)
   const MfmaWeightPlan mp = weight_mfma_plan(g, true);
   const uint64_t mbytes = mp.lds_bytes > 0 && mp.chunks > 1 ? mp.chunks * mp.f.stride * 4ull : 0;
-  const LdsPlan lp = weight_lds_plan(g);
-  if (lp.tile > 0) {
-    const uint64_t lbytes = lp.chunks > 1 ? lp.chunks * (weight_elems(g) + g.out_c) * 4 : 0;
-    return lbytes > mbytes ? lbytes : mbytes;
-  }
-  if (mp.lds_bytes > 0) {
-    const uint64_t generic = weight_elems(g) * weight_chunks(g) * 4;
-    return generic > mbytes ? generic : mbytes;
-  }
   if (pointwise(g)) {
     const KSplit k = product_split(g);
     return k.chunks > 1 ? static_cast<uint64_t>(k.chunks) * g.out_c * g.in_c * 4 : 0;
   }
-  return weight_elems(g) * weight_chunks(g) * 4;
+  const uint32_t partials = large_weight_partials(g);
+  const LdsPlan lp = weight_lds_plan(g);
+  uint64_t bytes = weight_elems(g) * weight_chunks(g) * 4;
+  if (partials > 0)
+    bytes = partials > 1 ? weight_elems(g) * partials * 4 : 0;
+  else if (lp.tile > 0)
+    bytes = lp.chunks > 1 ? lp.chunks * (weight_elems(g) + g.out_c) * 4 : 0;
+  return bytes > mbytes ? bytes : mbytes;
 }
 
 oxh_status make_pool_geom(const char *name, const oxh_pool2d_shape *s, PoolGeom &g) {
@@ -3213,6 +3236,15 @@ oxh_status weight_backward_impl(const char *name, hipStream_t s, const ConvGeom 
                       mp.f.bias ? bias_gradient : nullptr);
     return oxh::launched(name);
   }
+  if (const uint32_t partials = large_weight_partials(g); partials > 0) {
+    oxh::conv_mfma::weight_backward(s, mfma_weight_dims(g), gradient, input,
+                                    partials > 1 ? partial : weight_gradient);
+    const oxh_status st = oxh::launched(name);
+    if (st != OXH_OK || partials == 1) return st;
+    launch_sum_chunks(s, static_cast<uint32_t>(weight_elems(g)), partials, partial,
+                      weight_gradient);
+    return oxh::launched(name);
+  }
   // the bias sums ride along where their threads fit; else the caller forms the bias
   bool bias = bias_gradient != nullptr && weight_lds_plan(g, true).tile > 0;
   const LdsPlan lp = weight_lds_plan(g, bias);
@@ -3247,8 +3279,8 @@ oxh_status weight_backward_impl(const char *name, hipStream_t s, const ConvGeom 
     launch_sum_chunks(s, stride, lp.chunks, partial, weight_gradient, weights, bias_gradient);
     return oxh::launched(name);
   }
-  const uint32_t chunks = weight_chunks(g);
   const uint32_t weights = static_cast<uint32_t>(weight_elems(g));
+  const uint32_t chunks = weight_chunks(g);
   oxh::launch(conv2d_weight_partial_kernel,
               dim3(grid_for(static_cast<uint64_t>(weights) * chunks)), dim3(256), 0, s, g,
               weights, oxh::make_fastdiv(weights), chunks, gradient, input, partial);

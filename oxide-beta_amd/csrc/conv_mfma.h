@@ -28,5 +28,15 @@ void forward(hipStream_t s, const Dims &d, const float *x, const float *weight,
 void input_backward(hipStream_t s, const Dims &d, const float *gradient, const float *weight,
                     const float *addend, float *dx);
 
+// Weight gradient of an ungrouped convolution with any kernel.
+struct WeightDims {
+  uint32_t batch, in_c, h, w, out_c, kh, kw, stride, pad, oh, ow;
+};
+// Partial sums it leaves, each of out_c * in_c * kh * kw values (1: the gradient itself); 0 when
+// the shape does not run here.
+uint32_t weight_partials(const WeightDims &d);
+void weight_backward(hipStream_t s, const WeightDims &d, const float *gradient, const float *x,
+                     float *out);
+
 }  // namespace conv_mfma
 }  // namespace oxh

@@ -10,7 +10,8 @@ import torch
 
 import oracle
 import oxide_hip as ox
-from helpers import assert_conv_forward, assert_conv_input_gradient, host, to_dev
+from helpers import (assert_conv_forward, assert_conv_input_gradient, assert_within, host,
+                     to_dev)
 
 pytestmark = pytest.mark.gpu
 
@@ -91,3 +92,42 @@ def test_weights_that_are_not_finite(module, dev, case, value):
         np.testing.assert_allclose(got[fine], ref[fine], rtol=1e-4, atol=1e-4)
         assert np.array_equal(np.isnan(got), np.isnan(ref))
         assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+
+
+# batch, in, height, width, out, kernel, stride, padding: one to nine column tiles per block, one
+# and two row tiles, groups of one row and of several, image ends inside a group, widths padded
+# to eight positions, one partial sum
+WEIGHT_CASES = CASES + [
+    (1, 130, 9, 11, 33, 3, 1, 1),
+    (3, 64, 45, 44, 64, 3, 1, 1),
+    (2, 18, 50, 47, 40, 7, 3, 2),
+    (1, 2, 3, 300, 5, 3, 1, 1),
+    (4, 8, 18, 18, 32, 3, 1, 1),      # planes an LDS plan holds, over 64 positions
+]
+
+
+@pytest.mark.parametrize("case", WEIGHT_CASES)
+def test_weight_gradient(module, dev, case):
+    shape, x, wt, _, g = _case(case, dev)
+    dw = torch.full(wt.shape, float("nan"), device=dev)
+    module.conv2d_weight_backward(shape, to_dev(g, dev), to_dev(x, dev), dw)
+    ref = oracle.conv2d_backward(g, x, wt, case[6], case[7], 1)[1]
+    size = oracle.conv2d_backward(np.abs(g), np.abs(x), np.abs(wt), case[6], case[7], 1)[1]
+    assert_within(host(dw), ref, 1e-5 * size.astype(np.float64) + 1e-7, "weight gradient")
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("case", [(2, 33, 34, 31, 40, 3, 1, 1), (1, 30, 40, 44, 66, 3, 2, 1)])
+def test_gradients_that_are_not_finite(module, dev, case, value):
+    """An infinite or NaN output gradient in a corner reaches the weights whose tap lies inside
+    the input there, and no other."""
+    shape, x, wt, _, g = _case(case, dev)
+    g[0, 4, 0, 0] = value
+    dw = torch.empty(wt.shape, device=dev)
+    module.conv2d_weight_backward(shape, to_dev(g, dev), to_dev(x, dev), dw)
+    ref = oracle.conv2d_backward(g, x, wt, case[6], case[7], 1)[1]
+    fine = np.isfinite(ref)
+    assert (~fine).sum() == 4 * case[1]  # the corner's four taps of one output channel
+    assert np.array_equal(np.isnan(ref), np.isnan(host(dw)))
+    assert np.array_equal(host(dw)[np.isinf(ref)], ref[np.isinf(ref)])
+    np.testing.assert_allclose(host(dw)[fine], ref[fine], rtol=1e-3, atol=1e-3)
