@@ -1436,7 +1436,55 @@ __device__ __forceinline__ void bias_block(const BiasArgs &a, uint32_t b) {
   if (lane == 0) a.out[oc] = acc;
 }
 __global__ __launch_bounds__(256) void conv2d_bias_kernel(BiasArgs a) { bias_block(a, blockIdx.x); }
+// More than kWideBias terms per channel: a block of 1024 threads per channel, eight 128-bit loads
+// in flight per thread (scalar ones where planes are not whole float4s), fixed-order wave sums
+// added in wave order.  One wave per channel ran at the latency of its four loads in flight: 32
+// images of 64 x 56 x 56 took 131 us and now 8 us; 32 of 32 x 112 x 112, 547 us and now 22 us (32
+// blocks: bound by what one CU loads).  A channel's terms have to meet in one block, as the entry
+// point has no workspace.  The line is where a wave's dependent rounds of loads (6272 terms: 13 us
+// on the device) outlast the block's barrier and sums (4 us).  The paired 1 x 1 launch carries the
+// bias sums up to this many terms only, a wave per channel.
+constexpr uint32_t kWideBias = 4096;
+constexpr int kWideBiasThreads = 1024;
+template <bool Vec>
+__global__ __launch_bounds__(kWideBiasThreads) void conv2d_wide_bias_kernel(BiasArgs a) {
+  __shared__ float wave_sums[kWideBiasThreads / 64];
+  const uint32_t oc = blockIdx.x;
+  constexpr uint32_t V = Vec ? 4 : 1, U = 8;
+  const uint32_t total = a.batch * a.plane / V;  // loads; plane_div divides by plane / V
+  const uint32_t image = a.out_c * a.plane;
+  const float *g = a.grad + oc * a.plane;
+  float acc[1] = {0.0f};
+  for (uint32_t b = threadIdx.x; b < total; b += kWideBiasThreads * U) {
+    float4 v[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t e = b + u * kWideBiasThreads, i = e < total ? e : b;
+      const uint32_t n = fdiv(i, a.plane_div);
+      const float *at = g + static_cast<uint64_t>(n) * image + (i - n * a.plane_div.d) * V;
+      if constexpr (Vec)
+        v[u] = *reinterpret_cast<const float4 *>(at);
+      else
+        v[u] = make_float4(*at, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      if (b + u * kWideBiasThreads >= total) continue;
+      acc[0] += Vec ? (v[u].x + v[u].y) + (v[u].z + v[u].w) : v[u].x;
+    }
+  }
+  oxh::wave_sums_rows(acc);
+  if (threadIdx.x % 64 == 0) wave_sums[threadIdx.x / 64] = acc[0];
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  float sum = wave_sums[0];
+  for (int w = 1; w < kWideBiasThreads / 64; ++w) sum += wave_sums[w];
+  a.out[oc] = sum;
+}
 uint32_t bias_blocks(uint32_t out_c) { return (out_c + 3) / 4; }
+bool wide_bias(const ConvGeom &g) {
+  return static_cast<uint64_t>(g.batch) * g.oh * g.ow > kWideBias;
+}
 BiasArgs bias_args(const ConvGeom &g, const float *gradient, float *bias_gradient) {
   return BiasArgs{gradient, bias_gradient, g.batch, g.out_c, g.oh * g.ow,
                   oxh::make_fastdiv(g.oh * g.ow)};
@@ -3458,8 +3506,16 @@ oxh_status oxh_conv2d_bias_backward(oxh_stream stream, const oxh_conv2d_shape *s
   OXH_REQUIRE(gradient && bias_gradient, OXH_INVALID_SHAPE, std::string(name) + ": null pointer");
   (void)workspace;  // the single-pass reduction needs none
   (void)workspace_bytes;
-  oxh::launch(conv2d_bias_kernel, dim3(bias_blocks(g.out_c)), dim3(256), 0,
-              oxh::as_stream(stream), bias_args(g, gradient, bias_gradient));
+  BiasArgs a = bias_args(g, gradient, bias_gradient);
+  hipStream_t s = oxh::as_stream(stream);
+  if (!wide_bias(g)) {
+    oxh::launch(conv2d_bias_kernel, dim3(bias_blocks(g.out_c)), dim3(256), 0, s, a);
+  } else if (a.plane % 4 == 0 && oxh::aligned16(gradient)) {
+    a.plane_div = oxh::make_fastdiv(a.plane / 4);
+    oxh::launch(conv2d_wide_bias_kernel<true>, dim3(g.out_c), dim3(kWideBiasThreads), 0, s, a);
+  } else {
+    oxh::launch(conv2d_wide_bias_kernel<false>, dim3(g.out_c), dim3(kWideBiasThreads), 0, s, a);
+  }
   return oxh::launched(name);
 }
 
@@ -3513,12 +3569,15 @@ oxh_status oxh_conv2d_backward(oxh_stream stream, const oxh_conv2d_shape *shape,
     const ProductArgs w =
         weight_product(g, split, gradient, input, split.chunks > 1 ? partial : weight_gradient);
     const ProductArgs x = input_product(g, gradient, weight, addend, input_gradient);
-    if (launch_dual(s, w, split, x, bias_args(g, gradient, bias_gradient))) {
+    const bool wide = bias_gradient != nullptr && wide_bias(g);
+    if (launch_dual(s, w, split, x, bias_args(g, gradient, wide ? nullptr : bias_gradient))) {
       st = oxh::launched(name);
-      if (st != OXH_OK || split.chunks == 1) return st;
-      const uint32_t count = g.out_c * g.in_c;
-      launch_sum_chunks(s, count, split.chunks, partial, weight_gradient);
-      return oxh::launched(name);
+      if (st == OXH_OK && split.chunks > 1) {
+        launch_sum_chunks(s, g.out_c * g.in_c, split.chunks, partial, weight_gradient);
+        st = oxh::launched(name);
+      }
+      if (st != OXH_OK || !wide) return st;
+      return oxh_conv2d_bias_backward(stream, shape, gradient, bias_gradient, nullptr, 0);
     }
   }
   // a stride-2 K x K convolution whose two gradients both take the matrix-core kernels: one

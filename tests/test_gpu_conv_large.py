@@ -131,3 +131,40 @@ def test_gradients_that_are_not_finite(module, dev, case, value):
     assert np.array_equal(np.isnan(ref), np.isnan(host(dw)))
     assert np.array_equal(host(dw)[np.isinf(ref)], ref[np.isinf(ref)])
     np.testing.assert_allclose(host(dw)[fine], ref[fine], rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("batch,channels,height,width", [
+    (1, 3, 64, 64),      # the most terms a wave sums
+    (1, 3, 63, 67),      # a block per channel, scalar loads
+    (5, 7, 60, 56),      # float4s, a last round that is not full
+    (300, 33, 8, 8),     # many short planes
+])
+def test_bias_gradient(module, dev, batch, channels, height, width):
+    r = np.random.default_rng(batch)
+    g = r.standard_normal((batch, channels, height, width)).astype(np.float32)
+    shape = ox.conv2d_shape(batch, 2, height, width, channels, 3, 1, 1, 1)
+    db = torch.full((channels,), float("nan"), device=dev)
+    flat = torch.empty(g.size + 1, device=dev)
+    for lead in (0, 1):  # aligned, and one float past it
+        gd = flat[lead:lead + g.size].view(g.shape)
+        gd.copy_(torch.from_numpy(g))
+        module.conv2d_bias_backward(shape, gd, db)
+        assert_within(host(db), g.astype(np.float64).sum((0, 2, 3)),
+                      1e-5 * np.abs(g).astype(np.float64).sum((0, 2, 3)), "bias gradient")
+
+
+def test_paired_backward_leaves_wide_bias_sums_to_their_kernel(module, dev):
+    """A 1 x 1 backward whose two products share a launch, with more bias terms than a wave sums:
+    the bias equals the separate entry point's, bit for bit."""
+    r = np.random.default_rng(5)
+    shape = ox.conv2d_shape(110, 16, 7, 7, 16, 1, 1, 0, 1)
+    x = to_dev(r.standard_normal((110, 16, 7, 7)).astype(np.float32), dev)
+    g = to_dev(r.standard_normal((110, 16, 7, 7)).astype(np.float32), dev)
+    wt = to_dev(r.standard_normal((16, 16, 1, 1)).astype(np.float32), dev)
+    dx, dw = torch.empty_like(x), torch.empty_like(wt)
+    db, ref = (torch.full((16,), float("nan"), device=dev) for _ in range(2))
+    module.conv2d_backward(shape, g, x, wt, dx, dw, db)
+    module.conv2d_bias_backward(shape, g, ref)
+    assert np.array_equal(host(db), host(ref))
+    assert_within(host(db), host(g).astype(np.float64).sum((0, 2, 3)),
+                  1e-5 * np.abs(host(g)).astype(np.float64).sum((0, 2, 3)), "bias gradient")
