@@ -28,6 +28,14 @@ void forward(hipStream_t s, const Dims &d, const float *x, const float *weight,
 void input_backward(hipStream_t s, const Dims &d, const float *gradient, const float *weight,
                     const float *addend, float *dx);
 
+// A 1 x 1 convolution as a product: y[n][m][p] = bias[m] + sum over k of w[m][k] x[n][k][p] +
+// addend (bias and addend may be null, addend may be y), with w[m][k] at weight[m * k_count + k]
+// or, transposed (an input gradient: k the output channels), weight[k * m_count + m].
+bool takes_pointwise(uint64_t images, uint64_t plane, uint64_t k, uint64_t m);
+void pointwise(hipStream_t s, uint32_t images, uint32_t plane, uint32_t k, uint32_t m,
+               bool transposed, const float *x, const float *weight, const float *bias,
+               const float *addend, float *y);
+
 // Weight gradient of an ungrouped convolution with any kernel.
 struct WeightDims {
   uint32_t batch, in_c, h, w, out_c, kh, kw, stride, pad, oh, ow;

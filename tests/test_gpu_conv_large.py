@@ -168,3 +168,45 @@ def test_paired_backward_leaves_wide_bias_sums_to_their_kernel(module, dev):
     assert np.array_equal(host(db), host(ref))
     assert_within(host(db), host(g).astype(np.float64).sum((0, 2, 3)),
                   1e-5 * np.abs(host(g)).astype(np.float64).sum((0, 2, 3)), "bias gradient")
+
+
+# 1 x 1 layers, batch, in, height, width, out: pairs of positions (even planes, two blocks per
+# CU), single ones (odd planes; few blocks), four waves per position; ragged rows, positions
+# and channel chunks (16, 32 and 128 channels); a plane of 64 in a layer of over 2^27 products
+POINTWISE = [
+    (15, 37, 60, 150, 33), (16, 40, 93, 91, 70), (5, 33, 31, 13, 50), (3, 129, 11, 9, 40),
+    (1, 70, 9, 9, 5), (1, 200, 13, 6, 96), (6, 400, 10, 8, 130), (40, 130, 8, 8, 416),
+]
+
+
+@pytest.mark.parametrize("case", POINTWISE)
+@pytest.mark.parametrize("lead", [0, 1])
+def test_pointwise(module, dev, case, lead):
+    """Forward, input gradient and the input gradient added in place; with tensors one float past
+    their allocation's alignment (lead 1) too."""
+    n, cin, h, w, cout = case
+    r = np.random.default_rng(cin * cout + lead)
+    shape = ox.conv2d_shape(n, cin, h, w, cout, 1, 1, 0, 1)
+    assert not ox.conv2d_forward_serial(shape) and not ox.conv2d_input_backward_serial(shape)
+
+    def device(a):
+        flat = torch.empty(a.size + lead, device=dev)[lead:].view(a.shape)
+        return flat.copy_(torch.from_numpy(a))
+
+    x = r.standard_normal((n, cin, h, w)).astype(np.float32)
+    wt = (r.standard_normal((cout, cin, 1, 1)) * 0.3).astype(np.float32)
+    b = r.standard_normal(cout).astype(np.float32)
+    g = r.standard_normal((n, cout, h, w)).astype(np.float32)
+    xd, wd, gd = device(x), device(wt), device(g)
+    y, dx, summed = device(np.full_like(g, np.nan)), device(np.full_like(x, np.nan)), device(x)
+    module.conv2d_forward(shape, xd, wd, device(b), y)
+    module.conv2d_input_backward(shape, gd, wd, dx)
+    module.conv2d_input_backward_accumulate(shape, gd, wd, summed, summed)
+    matrix = wt.reshape(cout, cin).astype(np.float64)
+    for got, m, v, add in ((y, matrix, x, b[:, None, None]), (dx, matrix.T, g, 0.0),
+                           (summed, matrix.T, g, x)):
+        flat = v.reshape(n, v.shape[1], -1).astype(np.float64)
+        shaped = (n, m.shape[0], h, w)
+        ref = (m @ flat).reshape(shaped) + add
+        size = (np.abs(m) @ np.abs(flat)).reshape(shaped) + np.abs(add)
+        assert_within(host(got), ref, 1e-5 * size, "1 x 1")
