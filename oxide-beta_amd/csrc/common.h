@@ -24,6 +24,16 @@ oxh_status bn_scratch_init(int device);
 // sums the input gradient per channel in passing: a preceding convolution's bias gradient).
 bool batch_norm_single_launch(uint64_t batch, uint64_t channels, uint64_t spatial);
 
+// BatchNorm from the running statistics (inverse_std, output) and the elementwise op behind it
+// (tail_output = relu(output) or output + addend) in one launch; each value as
+// oxh_batch_norm_running_inverse_std, oxh_batch_norm_apply and oxh_relu / oxh_add form it.
+enum class EvalTail { None, Relu, Add };
+oxh_status batch_norm_eval(hipStream_t stream, uint64_t batch, uint64_t channels,
+                           uint64_t spatial, float epsilon, const float *input,
+                           const float *weight, const float *bias, const float *mean,
+                           const float *variance, float *inverse_std, float *output,
+                           EvalTail tail, const float *addend, float *tail_output);
+
 // One weight-gradient chunk sum: out[e] (e < split) or out2[e - split] (split <= e < count)
 // = the fixed-order sum over `chunks` of partial[chunk * count + e].
 struct ChunkSum {

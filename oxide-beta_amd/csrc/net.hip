@@ -423,6 +423,47 @@ OpRec bn_eval_forward_op(const Graph &g, const std::vector<float *> &value, floa
   return op;
 }
 
+// What the whole program runs for that group: one launch that also forms the value of `tail`
+// (bn_eval_tail's answer, or -1), whose own group then has nothing left to do.  Every value is
+// stored, bit for bit as the groups one by one leave it.
+std::function<oxh_status(hipStream_t)> bn_eval_program_launch(const Graph &g,
+                                                              const std::vector<float *> &value,
+                                                              float *inv, size_t i, int tail) {
+  const Node &x = g.nodes[i];
+  const float *xi = value[x.in[0]], *w = value[x.in[1]], *b = value[x.in[2]];
+  float *out = value[i], *rm = x.running_mean, *rv = x.running_variance;
+  const uint64_t N = x.shape[0], C = x.shape[1], HW = x.shape[2] * x.shape[3];
+  const float eps = x.epsilon;
+  oxh::EvalTail kind = oxh::EvalTail::None;
+  const float *addend = nullptr;
+  float *z = nullptr;
+  if (tail >= 0) {
+    const Node &t = g.nodes[tail];
+    z = value[tail];
+    kind = t.op == Op::Relu ? oxh::EvalTail::Relu : oxh::EvalTail::Add;
+    if (t.op == Op::Add) addend = value[t.in[0] == static_cast<int>(i) ? t.in[1] : t.in[0]];
+  }
+  return [=](hipStream_t st) {
+    return oxh::batch_norm_eval(st, N, C, HW, eps, xi, w, b, rm, rv, inv, out, kind, addend, z);
+  };
+}
+
+// The first ReLU of BatchNorm node i, or addition of it and a value that exists by then, not
+// taken by another BatchNorm; -1: none.
+int bn_eval_tail(const Graph &g, const std::vector<char> &active, const std::vector<char> &taken,
+                 size_t i) {
+  const int self = static_cast<int>(i);
+  for (size_t t = i + 1; t < g.nodes.size(); ++t) {
+    const Node &n = g.nodes[t];
+    if (!active[t] || taken[t]) continue;
+    if (n.op == Op::Relu && n.in[0] == self) return static_cast<int>(t);
+    if (n.op == Op::Add && (n.in[0] == self) != (n.in[1] == self) &&
+        (n.in[0] == self ? n.in[1] : n.in[0]) < self)
+      return static_cast<int>(t);
+  }
+  return -1;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------- forward program
@@ -467,6 +508,7 @@ oxh_status build_forward(const Graph &g, int output, oxh_program &p) {
   p.root = output;
   void *ws = a.at<void>(ws_off);
   const uint64_t wsb = ws_bytes;
+  std::vector<char> formed(n, 0);  // values an inference BatchNorm's launch forms with its own
   for (size_t i = 0; i < n; ++i) {
     const Node &x = g.nodes[i];
     if (!active[i] || x.leaf() || is_view(g, x)) continue;
@@ -478,13 +520,18 @@ oxh_status build_forward(const Graph &g, int output, oxh_program &p) {
       case Op::Add:
       case Op::Mul:
         p.ops.push_back(elementwise_forward_op(g, p.value, i));
+        if (formed[i]) p.ops.back().program_launch = [](hipStream_t) { return oxh::ok(); };
         break;
       case Op::Pool:
         p.ops.push_back(pool_forward_op(g, p.value, i));
         break;
       case Op::Bn: {
         if (!x.training) {
-          p.ops.push_back(bn_eval_forward_op(g, p.value, p.saved_inv[i], i));
+          OpRec op = bn_eval_forward_op(g, p.value, p.saved_inv[i], i);
+          const int tail = bn_eval_tail(g, active, formed, i);
+          if (tail >= 0) formed[tail] = 1;
+          op.program_launch = bn_eval_program_launch(g, p.value, p.saved_inv[i], i, tail);
+          p.ops.push_back(std::move(op));
           break;
         }
         // evaluation.rs:448-558: batch statistics, running update, apply

@@ -1,0 +1,68 @@
+"""Inference programs run whole (BatchNorm and the op behind it in one launch) against their
+launch groups run one by one: every node's value bit for bit."""
+
+import numpy as np
+import pytest
+import torch
+
+import nn
+import tensor as tn
+from helpers import host
+
+pytestmark = pytest.mark.gpu
+
+
+def _norm(channels, r):
+    bn = nn.BatchNorm2d(channels)
+    bn.set_training(False)
+    dev = bn.weight.data.device
+    for t, low, high in ((bn.weight.data, 0.5, 1.5), (bn.bias.data, -0.5, 0.5),
+                         (bn.state.running_mean, -0.3, 0.3),
+                         (bn.state.running_variance, 0.5, 2.0)):
+        t.copy_(torch.from_numpy(r.uniform(low, high, channels).astype(np.float32)).to(dev))
+    return bn
+
+
+@pytest.mark.parametrize("height,width", [(6, 6), (5, 7), (1, 1), (40, 52)])
+def test_whole_program_equals_its_groups(dev, height, width):
+    """A ReLU behind, an addition behind (either operand order), nothing behind, a BatchNorm with
+    both, an addition whose other operand comes later, and one of a value to itself."""
+    r = np.random.default_rng(height * width)
+    c = 5
+    x = tn.input((3, c, height, width))
+    norms = [_norm(c, r) for _ in range(6)]
+    a = norms[0](x)
+    b = a.relu()
+    d = norms[1](nn.Conv2d(c, c, 1)(b))
+    e = b.add(d)                    # the other operand first, and before the BatchNorm
+    f = norms[2](e)
+    g = f.mul(e)                    # nothing to take in
+    h = norms[3](g)
+    i, j = h.relu(), h.add(e)       # both: the ReLU goes along
+    k = norms[4](j)
+    m = k.add(nn.Conv2d(c, c, 1)(i))  # the convolution runs after the BatchNorm
+    o = norms[5](m)
+    out = o.add(o)
+    nodes = [a, b, d, e, f, g, h, i, j, k, m, o, out]
+    program = tn.forward_program(out, [x])
+    program.feed(x, r.standard_normal((3, c, height, width)).astype(np.float32))
+    kinds = [op.kind for op in program.ops]
+    assert kinds.count("batch_norm2d_eval_forward") == 6
+    for op in program.ops:
+        op.launch()
+    program.synchronize()
+    one_by_one = [program.value(t).host() for t in nodes]
+    for t in nodes:
+        program.value(t).copy_from(np.full(t.shape, np.nan, np.float32))
+    program.run()
+    program.synchronize()
+    whole = [program.value(t).host() for t in nodes]
+    program.capture()
+    for t in nodes:
+        program.value(t).copy_from(np.full(t.shape, np.nan, np.float32))
+    program.replay()
+    program.synchronize()
+    replayed = [program.value(t).host() for t in nodes]
+    for t, p, q, s in zip(nodes, one_by_one, whole, replayed):
+        assert np.isfinite(p).all()
+        assert np.array_equal(p, q) and np.array_equal(p, s), t
