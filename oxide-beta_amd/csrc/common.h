@@ -20,8 +20,8 @@ namespace oxh {
 // forward's partials); `device` must be current.  Called by oxh_init.
 oxh_status bn_scratch_init(int device);
 
-// Whether a training BatchNorm of this shape runs one block per channel (its backward then
-// sums the input gradient per channel in passing: a preceding convolution's bias gradient).
+// Whether a training BatchNorm of this shape runs one block per channel and its backward should
+// also sum the input gradient per channel in passing (a preceding convolution's bias gradient).
 bool batch_norm_single_launch(uint64_t batch, uint64_t channels, uint64_t spatial);
 
 // BatchNorm from the running statistics (inverse_std, output) and the elementwise op behind it

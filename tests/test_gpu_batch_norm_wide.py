@@ -1,0 +1,87 @@
+"""BatchNorm training forward and backward with one block per channel over planes of 64 values and
+more, against the oracle at the edges of its units (planes of 4 n + 0 .. 3 values, one to eight
+units per thread, 256 and 1024 threads, the shapes just past them)."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import (assert_within, check_batch_norm_backward, check_batch_norm_forward, host,
+                     to_dev)
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    (2, 3, 8, 8),       # the smallest plane
+    (5, 70, 5, 13),     # planes of 4 n + 1 values
+    (3, 66, 13, 10),    # 4 n + 2
+    (23, 65, 9, 11),    # 4 n + 3: 575 units, two per thread of 1024
+    (16, 2, 8, 16),     # 512 units: two per thread of 256
+    (19, 72, 35, 35),   # eight units per thread, the last ones partly idle
+    (8, 64, 64, 64),    # 8192 units: every thread full
+    (8, 64, 64, 65),    # past them: reduce and map
+    (4, 5, 64, 64),     # few channels: 4096 units
+    (4, 5, 64, 66),     # past them
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("lead", [0, 1])
+def test_training_step(module, dev, shape, lead):
+    """Forward and backward, alone, with the ReLU behind, with a residual addition and with the
+    input gradient's channel sums; tensors at their allocation's start and one float past it."""
+    n, c, h, w = shape
+    r = np.random.default_rng(n * c * h * w)
+    x = (r.standard_normal(shape) * 1.3 + 0.4).astype(np.float32)
+    g, more = (r.standard_normal(shape).astype(np.float32) for _ in range(2))
+    gamma = r.uniform(0.5, 1.5, c).astype(np.float32)
+    beta = r.uniform(-0.1, 0.1, c).astype(np.float32)
+    rm = r.uniform(-0.5, 0.5, c).astype(np.float32)
+    rv = r.uniform(0.5, 2.0, c).astype(np.float32)
+
+    def device(a=None):
+        flat = torch.full((x.size + lead,), float("nan"), device=dev)[lead:].view(shape)
+        return flat if a is None else flat.copy_(torch.from_numpy(a))
+
+    xd, gd, mored = device(x), device(g), device(more)
+    vec = lambda: torch.full((c,), float("nan"), device=dev)  # noqa: E731
+    wd, bd = to_dev(gamma, dev), to_dev(beta, dev)
+    out = {}
+    for kind in ("plain", "relu", "add"):
+        rmd, rvd, mean, inv, y = to_dev(rm, dev), to_dev(rv, dev), vec(), vec(), device()
+        args = (xd, wd, bd, rmd, rvd, mean, inv)
+        if kind == "plain":
+            module.batch_norm_forward_train(*args, y)
+        elif kind == "relu":
+            module.batch_norm_relu_forward_train(*args, y)
+        else:
+            module.batch_norm_add_forward_train(*args, mored, y)
+        out[kind] = dict(y=host(y), mean=host(mean), inv=host(inv), rm=host(rmd), rv=host(rvd))
+    check_batch_norm_forward(out["plain"], x, gamma, beta, rm, rv)
+    for k in ("mean", "inv", "rm", "rv"):
+        assert np.array_equal(out["plain"][k], out["relu"][k])
+        assert np.array_equal(out["plain"][k], out["add"][k])
+    assert np.array_equal(out["relu"]["y"], oracle.relu(out["plain"]["y"]))
+    assert np.array_equal(out["add"]["y"], out["plain"]["y"] + more)
+
+    mean, inv = out["plain"]["mean"], out["plain"]["inv"]
+    md, id = to_dev(mean, dev), to_dev(inv, dev)
+    relu_y = device(out["relu"]["y"])
+    masked = oracle.relu_backward(g, out["plain"]["y"])
+    for relu in (None, relu_y):
+        incoming = g if relu is None else masked
+        dx, dw, db, total = device(), vec(), vec(), vec()
+        if relu is None:
+            module.batch_norm_backward_train(gd, xd, wd, md, id, dx, dw, db)
+        else:
+            module.batch_norm_relu_backward_train(gd, relu, xd, wd, md, id, dx, dw, db)
+        got = dict(dx=host(dx), dw=host(dw), db=host(db))
+        check_batch_norm_backward(got, incoming, x, gamma, mean, inv)
+        summed, dw2, db2 = device(), vec(), vec()
+        module.conv_batch_norm_backward_train(gd, relu, xd, wd, md, id, summed, dw2, db2, total)
+        for a, b in ((summed, "dx"), (dw2, "dw"), (db2, "db")):
+            assert np.array_equal(host(a), got[b])
+        wide = got["dx"].astype(np.float64)
+        assert_within(host(total), wide.sum((0, 2, 3)),
+                      1e-6 * np.abs(wide).sum((0, 2, 3)) + 1e-7, "input gradient sums")
