@@ -793,12 +793,12 @@ __global__ __launch_bounds__(Threads) void bn_channel_backward_kernel(
 }
 
 // Larger planes of up to kWideUnits four-value units per channel: one block of 1024 threads (256
-// up to 512 units) per channel, the channel's values (Q units per thread) held in registers between the sums and the
-// elementwise pass.  One launch and one read of each tensor in place of a reduce and a map launch
-// with two; bound by what one CU loads and by the block's two phases.  Replayed alone, forward /
-// backward: 32 images of 192 x 14 x 14 10.2 / 9.3 -> 5.0 / 4.7 us, of 192 x 28 x 28 13.2 / 18.1 ->
-// 9.0 / 11.1 us, and with the input gradient's channel sums (a convolution's bias gradient)
-// 17.4 -> 5.3 us and 25.8 -> 11.7 us.
+// up to 512 units) per channel, the channel's values (Q units per thread) held in registers between
+// the sums and the elementwise pass.  One launch and one read of each tensor in place of a reduce
+// and a map launch with two; bound by what one CU loads and by the block's two phases.  Replayed
+// alone, forward / backward: 32 images of 192 x 14 x 14 10.2 / 9.3 -> 5.1 / 4.8 us, of
+// 192 x 28 x 28 13.2 / 18.1 -> 9.5 / 11.6 us, and with the input gradient's channel sums (a
+// convolution's bias gradient) 17.4 -> 5.4 us and 25.8 -> 12.2 us.
 constexpr int kWideThreads = 1024;
 constexpr uint32_t kWideUnits = kWideThreads * 8;
 

@@ -32,9 +32,10 @@
 //     1e-5 * sum|terms| of the CPU's serial sum.
 //   * Ungrouped K x K convolutions with small planes stage one image's planes and a channel
 //     tile's weights in LDS per block; larger ones run on the matrix cores over flattened
-//     positions (conv_mfma.hip); the rest (and depthwise convolutions not fused with
-//     their BatchNorm, depthwise_bn.hip) run one output (or input, or weight-chunk) element
-//     per thread.
+//     positions (conv_mfma.hip).
+//   * Depthwise convolutions not fused with their BatchNorm (depthwise_bn.hip) run in tiles of
+//     outputs per thread (conv_depthwise.hip); the rest run one output (or input, or
+//     weight-chunk) element per thread.
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -2859,8 +2860,8 @@ int input_splits(const ProductArgs &x) {
 
 // Pointwise forwards and input gradients on the matrix cores (conv_pointwise_mfma.hip): layers of
 // over 2^27 products, and planes of over 64 positions but for the small grids of many channels
-// that the split tiles take (8 images of 960 x 9 x 9 to 33 channels: 8.6 us, against 18 us for the
-// chunked walk over the channels there).  Smaller layers keep the CPU path's order.
+// that the split tiles take (8 images of 960 x 9 x 9 to 33 channels: 8.6 us, against 15 us for the
+// channel split there).  Smaller layers keep the CPU path's order.
 bool large_pointwise(const ConvGeom &g, bool forward) {
   if (!pointwise(g)) return false;
   const uint32_t plane = g.h * g.w, m = forward ? g.out_c : g.in_c, k = forward ? g.in_c : g.out_c;
@@ -2935,6 +2936,18 @@ bool depthwise_single_pass(const ConvGeom &g) {
          (g.kh == 3 || g.kh == 5) && g.out_c <= 65535 * 16;
 }
 
+// Those of them with four and more columns run in tiles (conv_depthwise.hip): as fast at the
+// smallest (8 images of 72 x 4 x 4: 7 to 9 us both ways, the launch) and up to ten times as fast
+// at the largest.  The weight gradient of a 3 x 3 kernel at stride 2 keeps a thread per position up
+// to 64 of them, where half of each tile's loads would be for nothing (32 images of 576 x 14 x 14:
+// 10.1 against 13.4 us; 96 x 56 x 56: 39 against 21 us).
+bool tiled_depthwise(const ConvGeom &g) {
+  return depthwise_single_pass(g) && oxh::conv_mfma::takes_depthwise(mfma_dims(g));
+}
+bool tiled_depthwise_weight(const ConvGeom &g) {
+  return tiled_depthwise(g) && !(g.kh == 3 && g.stride == 2 && g.oh * g.ow <= 64);
+}
+
 // Ungrouped weight gradients the per-image matrix-core kernel (weight_mfma_plan) does not take run
 // on the matrix cores over groups of output rows (conv_weight_mfma.hip), but for short serial
 // sums: planes of at most 64 positions with an LDS plan (33 images of 5 x 7 x 7 to 9 channels:
@@ -2955,6 +2968,10 @@ uint32_t large_weight_partials(const ConvGeom &g) {
 }
 
 uint64_t weight_partial_bytes(const ConvGeom &g) {
+  if (tiled_depthwise_weight(g)) {
+    const uint32_t chunks = oxh::conv_mfma::depthwise_weight_partials(mfma_dims(g));
+    return chunks > 1 ? weight_elems(g) * chunks * 4 : 0;
+  }
   if (depthwise_single_pass(g)) return 0;
   // the per-image matrix-core kernel's chunks or, where it does not take the shape or the operands'
   // alignment, the larger of those and the partial sums of the kernel that then runs (the LDS
@@ -3178,6 +3195,11 @@ oxh_status input_backward_impl(const char *name, oxh_stream stream,
     const ProductArgs x = input_product(g, gradient, weight, addend, input_gradient);
     return launch_product(name, s, x, 1, input_splits(x) != 0);
   }
+  if (tiled_depthwise(g)) {
+    oxh::conv_mfma::depthwise_input_backward(s, mfma_dims(g), gradient, weight, addend,
+                                             input_gradient);
+    return oxh::launched(name);
+  }
   if (large_input_backward(g)) {
     oxh::conv_mfma::input_backward(s, mfma_dims(g), gradient, weight, addend, input_gradient);
     return oxh::launched(name);
@@ -3244,6 +3266,13 @@ oxh_status weight_backward_impl(const char *name, hipStream_t s, const ConvGeom 
     if (st != OXH_OK || split.chunks == 1) return st;
     const uint32_t count = g.out_c * g.in_c;
     launch_sum_chunks(s, count, split.chunks, partial, weight_gradient);
+    return oxh::launched(name);
+  }
+  if (tiled_depthwise_weight(g)) {
+    const uint32_t chunks = oxh::conv_mfma::depthwise_weight_partials(mfma_dims(g));
+    oxh::conv_mfma::depthwise_weight_backward(s, mfma_dims(g), gradient, input,
+                                              chunks > 1 ? partial : weight_gradient);
+    if (chunks > 1) launch_sum_chunks(s, weight_elems(g), chunks, partial, weight_gradient);
     return oxh::launched(name);
   }
   if (depthwise_single_pass(g)) {
@@ -3421,6 +3450,10 @@ oxh_status oxh_conv2d_forward(oxh_stream stream, const oxh_conv2d_shape *shape,
     a.K = g.in_c;
     a.k_chunk = a.K;
     return launch_product(name, s, a, 1, true);
+  }
+  if (tiled_depthwise(g)) {
+    oxh::conv_mfma::depthwise_forward(s, mfma_dims(g), input, weight, bias, output);
+    return oxh::launched(name);
   }
   if (large_forward(g)) {
     oxh::conv_mfma::forward(s, mfma_dims(g), input, weight, bias, output);

@@ -1,5 +1,5 @@
-// conv_mfma.h -- ungrouped square-kernel convolutions over large planes on the matrix cores
-// (internal to the library; conv.hip chooses).
+// conv_mfma.h -- square-kernel convolutions over large planes: ungrouped ones on the matrix cores,
+// depthwise ones in tiles (internal to the library; conv.hip chooses).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -45,6 +45,18 @@ struct WeightDims {
 uint32_t weight_partials(const WeightDims &d);
 void weight_backward(hipStream_t s, const WeightDims &d, const float *gradient, const float *x,
                      float *out);
+
+// Depthwise convolutions (in_c == out_c == groups) with kernel 3 or 5 and stride 1 or 2
+// (conv_depthwise.hip).  addend as in input_backward.
+bool takes_depthwise(const Dims &d);
+void depthwise_forward(hipStream_t s, const Dims &d, const float *x, const float *weight,
+                       const float *bias, float *y);
+void depthwise_input_backward(hipStream_t s, const Dims &d, const float *gradient,
+                              const float *weight, const float *addend, float *dx);
+// Partial sums the weight gradient leaves, each of in_c * k * k values (1: the gradient itself).
+uint32_t depthwise_weight_partials(const Dims &d);
+void depthwise_weight_backward(hipStream_t s, const Dims &d, const float *gradient,
+                               const float *x, float *out);
 
 }  // namespace conv_mfma
 }  // namespace oxh
