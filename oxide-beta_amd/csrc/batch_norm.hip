@@ -991,7 +991,9 @@ __global__ void bn_running_inverse_std_kernel(uint32_t channels, float epsilon,
 // Inference: the channel's inverse deviation, BatchNorm from the running statistics and the op
 // behind it (Tail 1: z = relu(y), 2: z = y + addend, 0: none) in one pass, every value as the
 // separate launches form it and all of them stored (a program's values can be read at any
-// node).  V values per unit (float4s where planes are whole ones), two units per thread: the
+// node).  V values per unit (float4s where planes are whole ones, and with Cross where they are
+// not: a unit then may reach into the next plane and holds that channel's values too; the 7 x 7
+// layers of the network, batch 64, with a ReLU behind: 6.6 -> 6.1 us), two units per thread: the
 // channel's four values come from L1 and the square root and division, once per unit, stay under
 // the memory time.  In place of three launches reading and writing the activations twice: the 46
 // such layers of the 224 x 224 network, batch 64, take 770 us as separate launches and 359 us as
@@ -1001,19 +1003,22 @@ struct EvalArgs {
   float *inverse_std, *y, *z;
   float epsilon;
   uint32_t units, channels;
-  oxh::FastDiv spatial_div, channel_div;  // spatial in units
+  oxh::FastDiv spatial_div, channel_div;  // spatial in units (Cross: in values)
 };
-template <int V, int Tail>
+template <int V, int Tail, bool Cross = false>
 __global__ __launch_bounds__(kMapBlock) void bn_eval_kernel(EvalArgs a) {
   constexpr uint32_t U = 2;
   const uint32_t base = blockIdx.x * (kMapBlock * U) + threadIdx.x;
-  float x[U][V], add[U][V], w[U], b[U], mu[U], var[U];
-  uint32_t plane[U], at[U];
+  constexpr int P = Cross ? 2 : 1;  // planes of a unit
+  float x[U][V], add[U][V], w[U][P], b[U][P], mu[U][P], var[U][P];
+  uint32_t plane[U], at[U], left[U];  // left: the unit's values in its first plane
 #pragma unroll
   for (uint32_t u = 0; u < U; ++u) {
     const uint32_t q = base + u * kMapBlock;
     at[u] = q < a.units ? q : a.units - 1;
-    plane[u] = oxh::fast_div(at[u], a.spatial_div);
+    const uint32_t first = Cross ? V * at[u] : at[u];
+    plane[u] = oxh::fast_div(first, a.spatial_div);
+    left[u] = (plane[u] + 1) * a.spatial_div.d - first;
     const uint32_t c = plane[u] - oxh::fast_div(plane[u], a.channel_div) * a.channels;
     if constexpr (V == 4) {
       const float4 v = reinterpret_cast<const float4 *>(a.x)[at[u]];
@@ -1026,21 +1031,33 @@ __global__ __launch_bounds__(kMapBlock) void bn_eval_kernel(EvalArgs a) {
       x[u][0] = a.x[at[u]];
       if constexpr (Tail == 2) add[u][0] = a.addend[at[u]];
     }
-    w[u] = a.weight[c];
-    b[u] = a.bias[c];
-    mu[u] = a.mean[c];
-    var[u] = a.variance[c];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const uint32_t cp = p == 0 ? c : c + 1 < a.channels ? c + 1 : 0;
+      w[u][p] = a.weight[cp];
+      b[u][p] = a.bias[cp];
+      mu[u][p] = a.mean[cp];
+      var[u][p] = a.variance[cp];
+    }
   }
 #pragma unroll
   for (uint32_t u = 0; u < U; ++u) {
     const uint32_t q = base + u * kMapBlock;
     if (q >= a.units) return;
-    const float inv = 1.0f / sqrtf(var[u] + a.epsilon);
-    if (plane[u] < a.channels && q == plane[u] * a.spatial_div.d) a.inverse_std[plane[u]] = inv;
+    float inv[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) inv[p] = 1.0f / sqrtf(var[u][p] + a.epsilon);
+    if (plane[u] < a.channels && left[u] == a.spatial_div.d) a.inverse_std[plane[u]] = inv[0];
+    if constexpr (Cross) {  // the next plane starts inside the unit
+      if (left[u] < V && plane[u] + 1 < a.channels) a.inverse_std[plane[u] + 1] = inv[1];
+    }
     float y[V], z[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-      y[i] = (x[u][i] - mu[u]) * inv * w[u] + b[u];  // evaluation.rs:590-595
+      const bool next = Cross && static_cast<uint32_t>(i) >= left[u];
+      const float m = next ? mu[u][P - 1] : mu[u][0], s = next ? inv[P - 1] : inv[0];
+      const float wi = next ? w[u][P - 1] : w[u][0], bi = next ? b[u][P - 1] : b[u][0];
+      y[i] = (x[u][i] - m) * s * wi + bi;  // evaluation.rs:590-595
       if constexpr (Tail == 1) z[i] = y[i] > 0.0f ? y[i] : 0.0f;
       if constexpr (Tail == 2) z[i] = y[i] + add[u][i];
     }
@@ -1795,9 +1812,15 @@ oxh_status oxh::batch_norm_eval(hipStream_t stream, uint64_t batch, uint64_t cha
   const char *name = "batch_norm_eval";
   oxh_status st = check_shape(name, batch, channels, spatial);
   if (st != OXH_OK) return st;
-  const bool vec = spatial % 4 == 0 && oxh::aligned16(input) && oxh::aligned16(output) &&
-                   oxh::aligned16(addend) && oxh::aligned16(tail_output);
-  const uint64_t units = batch * channels * spatial / (vec ? 4 : 1);
+  const uint64_t values = batch * channels * spatial;
+  const bool quads = values % 4 == 0 && oxh::aligned16(input) && oxh::aligned16(output) &&
+                     oxh::aligned16(addend) && oxh::aligned16(tail_output);
+  const bool vec = quads && spatial % 4 == 0;
+  // planes of five values and more: a unit reaches over at most two; without an op behind, value
+  // by value is as fast (64 x 96 x 7 x 7: 4.7 against 4.9 us)
+  const bool cross =
+      quads && !vec && spatial > 4 && values < (1ull << 31) && tail != EvalTail::None;
+  const uint64_t units = values / (vec || cross ? 4 : 1);
   OXH_REQUIRE(units < (1ull << 31) - 2 * kMapBlock, OXH_INVALID_SHAPE,
               std::string(name) + ": tensors are limited to 2^31 elements");
   EvalArgs a{input, weight, bias, mean, variance, addend, inverse_std, output, tail_output,
@@ -1812,6 +1835,10 @@ oxh_status oxh::batch_norm_eval(hipStream_t stream, uint64_t batch, uint64_t cha
     oxh::launch(bn_eval_kernel<4, 2>, grid, block, 0, stream, a);
   else if (vec)
     oxh::launch(bn_eval_kernel<4, 0>, grid, block, 0, stream, a);
+  else if (cross && tail == EvalTail::Relu)
+    oxh::launch(bn_eval_kernel<4, 1, true>, grid, block, 0, stream, a);
+  else if (cross && tail == EvalTail::Add)
+    oxh::launch(bn_eval_kernel<4, 2, true>, grid, block, 0, stream, a);
   else if (tail == EvalTail::Relu)
     oxh::launch(bn_eval_kernel<1, 1>, grid, block, 0, stream, a);
   else if (tail == EvalTail::Add)

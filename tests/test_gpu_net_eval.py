@@ -66,3 +66,38 @@ def test_whole_program_equals_its_groups(dev, height, width):
     for t, p, q, s in zip(nodes, one_by_one, whole, replayed):
         assert np.isfinite(p).all()
         assert np.array_equal(p, q) and np.array_equal(p, s), t
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 4, 1, 5),    # the smallest plane a unit can leave
+    (4, 1, 3, 3),    # one channel: the next plane's channel is the same
+    (2, 6, 7, 7),    # a unit may start one to three values before a plane's end
+    (3, 4, 3, 5),    # planes of 4 n + 3 values
+    (1, 4, 3, 7),    # one image: every plane's inverse deviation is stored
+    (64, 96, 7, 7),  # many blocks
+    (3, 5, 5, 7),    # no whole number of units: value by value
+])
+def test_planes_of_no_whole_units(dev, shape):
+    """Units of four values that may reach into the next plane: nothing, a ReLU and an addition
+    behind, against the groups one by one."""
+    r = np.random.default_rng(sum(shape))
+    x = tn.input(shape)
+    a = _norm(shape[1], r)(x)
+    b = a.relu()
+    d = _norm(shape[1], r)(b)
+    e = d.add(a)
+    f = _norm(shape[1], r)(e)
+    program = tn.forward_program(f.mul(e), [x])
+    program.feed(x, r.standard_normal(shape).astype(np.float32))
+    for op in program.ops:
+        op.launch()
+    program.synchronize()
+    nodes = [a, b, d, e, f]
+    one_by_one = [program.value(t).host() for t in nodes]
+    for t in nodes:
+        program.value(t).copy_from(np.full(t.shape, np.nan, np.float32))
+    program.run()
+    program.synchronize()
+    for t, want in zip(nodes, one_by_one):
+        assert np.isfinite(want).all()
+        assert np.array_equal(program.value(t).host(), want), t
