@@ -400,11 +400,11 @@ oxh_status oxh_adamw_multi_tensor_table_step(oxh_stream stream, float learning_r
  * output tiles; ungrouped 3x3 / 5x5 with output planes of at most 64 positions and at least 16
  * input channels), and a pointwise input gradient with at least 256 output channels and fewer
  * than 512 32x32 tiles, sum four contiguous parts of the reduced channels and add the parts in
- * order; ungrouped 1x1 (strided or padded), 3x3 and 5x5 layers whose planes the per-image kernels
- * do not hold, or of over 2^27 products, sum on the matrix cores.  Those sums, and the weight and bias gradients
- * (fixed-order chunks), are deterministic and within a few roundings (1e-5 * sum|terms|) of
- * the serial sum; their products are added by fused multiply-adds (one rounding per term),
- * on the matrix cores (fp32 MFMA) for the split tiles and the 32x32 weight-gradient tiles. */
+ * order; ungrouped 1x1, 3x3 and 5x5 layers over larger planes, or of over 2^27 products, sum on
+ * the matrix cores.  Those sums, and the weight and bias gradients (fixed-order chunks), are
+ * deterministic and within a few roundings (1e-5 * sum|terms|) of the serial sum; their products
+ * are added by fused multiply-adds (one rounding per term), on the matrix cores (fp32 MFMA) for
+ * the split tiles and the 32x32 weight-gradient tiles. */
 typedef struct oxh_conv2d_shape {
   uint64_t batch, in_channels, height, width;
   uint64_t out_channels, kernel_h, kernel_w;
