@@ -11,6 +11,16 @@
 namespace oxh {
 namespace conv_mfma {
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// acc += a x b (v_mfma_f32_32x32x2_f32) in the lanes, columns of the result, that are `in`; the
+// others keep acc.
+__device__ __forceinline__ void multiply_in(float a, float b, bool in, f32x16 &acc) {
+  const f32x16 next = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = in ? next[r] : acc[r];
+}
+
 // One group, kernel k x k, the shape checks of conv.hip passed.
 struct Dims {
   uint32_t batch, in_c, h, w, out_c, k, stride, pad, oh, ow;

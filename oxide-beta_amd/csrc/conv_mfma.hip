@@ -20,8 +20,9 @@
 // within 1e-5 * sum|terms| of the CPU path's serial sum, and the same on every run.
 //
 // The CPU path skips a tap outside the plane; the +0 operand adds 0 * weight in its place, the
-// same for finite weights.  A block that meets an infinity or a NaN among its weights forms its
-// outputs again without the matrix cores, skipping those taps.
+// same for finite weights.  A block that meets an infinity or a NaN among its weights sums again
+// and keeps, at each product, the old sum in the columns whose tap lies outside (a lane holds one
+// column, so that is a select): 32 images of 64 x 56 x 56, 3 x 3, all weights NaN: 310 us.
 #include <hip/hip_runtime.h>
 
 #include "conv_mfma.h"
@@ -29,8 +30,6 @@
 namespace oxh {
 namespace conv_mfma {
 namespace {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kRows = 32;        // output channels of a block
 constexpr int kPositions = 128;  // its positions: 32 for each of its four waves
@@ -123,7 +122,7 @@ struct WeightStage {
 // pad = K - 1 - the convolution's, taps turned round, weights read as (source, output, tap)).
 // Block: 32 output channels x 128 positions, wave w the w-th 32 positions.
 template <int K, bool Flip, int CB>
-__global__ __launch_bounds__(256) void conv_taps_kernel(TapArgs g) {
+__global__ __launch_bounds__(256, K == 1 ? 8 : K == 3 ? 4 : 2) void conv_taps_kernel(TapArgs g) {
   constexpr int T = K * K, Pairs = CB / 2;
   using Stage = WeightStage<T, CB, Flip, Flip>;
   __shared__ float wl[2][CB * T * Stage::kRow];
@@ -152,11 +151,14 @@ __global__ __launch_bounds__(256) void conv_taps_kernel(TapArgs g) {
                 : kNowhere;
   }
   f32x16 acc;
+  auto start = [&](const float *bias) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const uint32_t m = m0 + tile_row(r, h);
-    acc[r] = g.bias != nullptr && m < g.M ? g.bias[m] : 0.0f;
-  }
+    for (int r = 0; r < 16; ++r) {
+      const uint32_t m = m0 + tile_row(r, h);
+      acc[r] = bias != nullptr && m < g.M ? bias[m] : 0.0f;
+    }
+  };
+  start(g.bias);
   // the pair of channels c, c + 1 at every tap (+0 past the channels)
   auto fetch = [&](uint32_t c, float (&b)[T]) {
     const uint32_t past = c + h < g.C ? 0u : kNowhere;
@@ -187,26 +189,24 @@ __global__ __launch_bounds__(256) void conv_taps_kernel(TapArgs g) {
     }
     if (more) odd |= ws.store(wl[buf ^ 1]);
   }
-  const bool direct = __syncthreads_or(odd) != 0;
+  if (__syncthreads_or(odd) != 0) {  // one product at a time, both operands from memory
+    const float *bias = g.bias;
+    asm volatile("" : "+s"(bias));  // loaded again, not held in registers over the sums
+    start(bias);
+    const uint32_t row = m0 + j < g.M ? ((m0 + j) * g.w_m + h * g.w_c) * 4u : kNowhere;
+#pragma unroll 1
+    for (uint32_t c = 0; c < g.C; c += 2) {
+      const uint32_t past = c + h < g.C ? 0u : kNowhere;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        multiply_in(load(wr, row | past, (c * g.w_c + (Flip ? T - 1 - t : t)) * 4u),
+                    load(xr, off[t] | past, c * plane * 4u), off[t] != kNowhere, acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
   if (pos >= g.N) return;
   const uint64_t at = static_cast<uint64_t>(n) * g.M * oplane + q;
-  if (direct) {
-    const float *xn = g.x + static_cast<uint64_t>(n) * image;
-    for (uint32_t r = h; r < kRows && m0 + r < g.M; r += 2) {
-      const uint32_t m = m0 + r;
-      float v = g.bias != nullptr ? g.bias[m] : 0.0f;
-      for (uint32_t c = 0; c < g.C; ++c)
-        for (int t = 0; t < T; ++t) {
-          const int iy = by + t / K, ix = bx + t % K;
-          if (static_cast<uint32_t>(iy) < g.H && static_cast<uint32_t>(ix) < g.W)
-            v = __builtin_fmaf(xn[static_cast<uint64_t>(c) * plane + iy * g.W + ix],
-                               g.w[m * g.w_m + c * g.w_c + (Flip ? T - 1 - t : t)], v);
-        }
-      const uint64_t o = at + static_cast<uint64_t>(m) * oplane;
-      g.y[o] = g.addend != nullptr ? v + g.addend[o] : v;
-    }
-    return;
-  }
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const uint32_t m = m0 + tile_row(r, h);
@@ -229,7 +229,7 @@ struct PhaseArgs {
 };
 
 template <int K, int CB>
-__global__ __launch_bounds__(256) void conv_input_s2_kernel(PhaseArgs p) {
+__global__ __launch_bounds__(256, K == 1 ? 8 : 2) void conv_input_s2_kernel(PhaseArgs p) {
   constexpr int T = K * K, Pairs = CB / 2, M2 = (K + 1) / 2, B = M2 * M2;
   constexpr int Ahead = Pairs % 4 == 0 && B <= 4 ? 4 : 2;  // operand register sets
   using Stage = WeightStage<T, CB, false, true>;
@@ -296,33 +296,27 @@ __global__ __launch_bounds__(256) void conv_input_s2_kernel(PhaseArgs p) {
     }
     if (more) odd |= ws.store(wl[buf ^ 1]);
   }
-  const bool direct = __syncthreads_or(odd) != 0;
-  if (pos >= g.N) return;
-  const uint32_t oplane = g.OH * g.OW;
-  if (direct) {
-    for (int f = 0; f < 4; ++f) {
-      const int y = 2 * static_cast<int>(a) + f / 2 - g.pad;
-      const int x = 2 * static_cast<int>(bcol) + f % 2 - g.pad;
-      if (static_cast<uint32_t>(y) >= g.OH || static_cast<uint32_t>(x) >= g.OW) continue;
-      for (uint32_t r = h; r < kRows && m0 + r < g.M; r += 2) {
-        const uint32_t m = m0 + r;
-        float v = 0.0f;
-        for (uint32_t c = 0; c < g.C; ++c)
-          for (int ky = f / 2; ky < K; ky += 2)
-            for (int kx = f % 2; kx < K; kx += 2) {
-              const int oy = static_cast<int>(a) - ky / 2, ox = static_cast<int>(bcol) - kx / 2;
-              if (static_cast<uint32_t>(oy) < g.H && static_cast<uint32_t>(ox) < g.W)
-                v = __builtin_fmaf(
-                    g.x[(static_cast<uint64_t>(n) * g.C + c) * plane + oy * g.W + ox],
-                    g.w[m * g.w_m + c * g.w_c + ky * K + kx], v);
-            }
-        const uint64_t o = (static_cast<uint64_t>(n) * g.M + m) * oplane +
-                           static_cast<uint32_t>(y) * g.OW + static_cast<uint32_t>(x);
-        g.y[o] = g.addend != nullptr ? v + g.addend[o] : v;
+  if (__syncthreads_or(odd) != 0) {  // as in conv_taps_kernel
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[f][r] = 0.0f;
+    const uint32_t row = m0 + j < g.M ? ((m0 + j) * g.w_m + h * g.w_c) * 4u : kNowhere;
+#pragma unroll 1
+    for (uint32_t c = 0; c < g.C; c += 2) {
+      const uint32_t past = c + h < g.C ? 0u : kNowhere;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const int ky = t / K, kx = t % K, i = (ky / 2) * M2 + kx / 2;
+        multiply_in(load(wr, row | past, (c * g.w_c + t) * 4u),
+                    load(xr, off[i] | past, c * plane * 4u), off[i] != kNowhere,
+                    acc[(ky % 2) * 2 + kx % 2]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    return;
   }
+  if (pos >= g.N) return;
+  const uint32_t oplane = g.OH * g.OW;
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
     const int y = 2 * static_cast<int>(a) + f / 2 - g.pad;

@@ -24,7 +24,6 @@ namespace oxh {
 namespace conv_mfma {
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 

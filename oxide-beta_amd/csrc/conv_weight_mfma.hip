@@ -19,7 +19,8 @@
 // Fused multiply-adds in a fixed order: within 1e-5 * sum|terms| of the CPU path's running sum,
 // the same on every run.  The CPU path skips taps outside the plane where these products have a
 // zero: the same for finite gradients; a block that meets an infinity or a NaN among its
-// gradients sums its chunk again without the matrix cores, skipping those taps.
+// gradients sums its chunk again, one position per product, and keeps the old sum in the columns
+// whose tap lies outside (a lane holds one column: a select).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,8 +32,6 @@
 namespace oxh {
 namespace conv_mfma {
 namespace {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kNowhere = 0x80000000u;  // past every buffer resource
 constexpr uint64_t kMaxBytes = 1ull << 31;
@@ -51,7 +50,7 @@ struct WeightArgs {
   uint32_t srows, pw;  // staged source rows and columns per channel
   uint32_t ps;         // floats between the staged channels
   uint32_t channels;   // staged channels of a block
-  uint32_t wm;         // row tiles of a block (1, 2 or 4); 4 / wm position parts
+  uint32_t wm;         // row tiles of a block (1 or 2); 4 / wm position parts
   uint32_t per_image, groups, per_chunk;  // groups
   uint32_t tiles, row_blocks, out_stride;
   FastDiv tiles_div, row_blocks_div, per_image_div, gpos_div, srows_pw_div, pw_div, ow_div,
@@ -178,45 +177,58 @@ __global__ __launch_bounds__(256, 2) void conv_weight_kernel(WeightArgs a) {
       }
     }
   }
-  const bool direct = __syncthreads_or(odd) != 0;
   float *out = a.out + static_cast<uint64_t>(chunk * parts + part) * a.out_stride;
-  if (direct) {  // part 0 takes the whole chunk
-    for (uint32_t c = j; c < 32 * CT && col0 + c < columns; c += 32) {
-      const uint32_t col = col0 + c, ic = fast_div(col, a.taps_div), tap = col - ic * a.taps;
-      const uint32_t ky = fast_div(tap, a.kw_div);
-      const int dy = static_cast<int>(ky) - a.pad;
-      const int dx = static_cast<int>(tap - ky * a.KW) - a.pad;
-      for (uint32_t r = h; r < 32; r += 2) {
-        const uint32_t m = m0 + 32 * wm + r;
-        if (m >= a.M) break;
-        float v = 0.0f;
-        for (uint32_t gi = first; part == 0 && gi < last; ++gi) {
-          const uint32_t n = fast_div(gi, a.per_image_div);
-          const uint32_t oy0 = (gi - n * a.per_image) * a.rows;
-          const float *gn = a.g + (static_cast<uint64_t>(n) * a.M + m) * oplane;
-          const float *xn = a.x + (static_cast<uint64_t>(n) * a.C + ic) * plane;
-          for (uint32_t oy = oy0; oy < min(oy0 + a.rows, a.OH); ++oy)
-            for (uint32_t ox = 0; ox < a.OW; ++ox) {
-              const int iy = static_cast<int>(oy * a.stride) + dy;
-              const int ix = static_cast<int>(ox * a.stride) + dx;
-              if (static_cast<uint32_t>(iy) < a.H && static_cast<uint32_t>(ix) < a.W)
-                v = __builtin_fmaf(gn[oy * a.OW + ox], xn[iy * static_cast<int>(a.W) + ix], v);
-            }
-        }
-        out[m * columns + col] = v;
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const uint32_t col = col0 + 32 * ct + j;
-    if (col >= columns) continue;
+  const auto store = [&](uint32_t col, const f32x16 &sums) {
+    if (col >= columns) return;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const uint32_t m = m0 + 32 * wm + 8u * (r / 4) + 4u * h + r % 4;
-      if (m < a.M) out[m * columns + col] = acc[ct][r];
+      if (m < a.M) out[m * columns + col] = sums[r];
     }
+  };
+  if (__syncthreads_or(odd) == 0) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) store(col0 + 32 * ct + j, acc[ct]);
+    return;
+  }
+  // a position per product and a column tile at a time, both operands from memory
+  const uint32_t m = m0 + 32 * wm + j;
+#pragma unroll 1
+  for (uint32_t c0 = col0; c0 < col0 + 32 * CT && c0 < columns; c0 += 32) {
+    const uint32_t col = min(c0 + j, columns - 1);
+    const uint32_t ic = fast_div(col, a.taps_div), tap = col - ic * a.taps;
+    const uint32_t ky = fast_div(tap, a.kw_div), kx = tap - ky * a.KW;
+    f32x16 sums = {};
+#pragma unroll 1
+    for (uint32_t gi = first; gi < last; ++gi) {
+      const uint32_t n = fast_div(gi, a.per_image_div);
+      const uint32_t oy0 = (gi - n * a.per_image) * a.rows;
+      const uint32_t count = min(a.rows, a.OH - oy0) * a.OW;
+      const __amdgpu_buffer_rsrc_t gr =
+          resource(a.g + static_cast<uint64_t>(n) * a.M * oplane,
+                   static_cast<uint64_t>(a.M) * oplane);
+      const __amdgpu_buffer_rsrc_t xr = resource(a.x + static_cast<uint64_t>(n) * a.C * plane,
+                                                 static_cast<uint64_t>(a.C) * plane);
+      constexpr uint32_t U = 4;  // positions in flight
+#pragma unroll 1
+      for (uint32_t p0 = part; p0 < count; p0 += U * parts) {
+        float gv[U], xv[U];
+        bool in[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+          const uint32_t p = p0 + u * parts, row = fast_div(p, a.ow_div);
+          const uint32_t iy = (oy0 + row) * a.stride + ky - static_cast<uint32_t>(a.pad);
+          const uint32_t ix = (p - row * a.OW) * a.stride + kx - static_cast<uint32_t>(a.pad);
+          in[u] = p < count && iy < a.H && ix < a.W;
+          const bool mine = h == 0 && p < count;  // the other half's position: +0 both
+          gv[u] = load(gr, mine && m < a.M ? (m * oplane + oy0 * a.OW + p) * 4u : kNowhere);
+          xv[u] = load(xr, mine && in[u] ? (ic * plane + iy * a.W + ix) * 4u : kNowhere);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) multiply_in(gv[u], xv[u], in[u], sums);
+      }
+    }
+    store(c0 + j, sums);
   }
 }
 

@@ -156,3 +156,20 @@ def check_batch_norm_backward(out, g, x, gamma, mean, inv):
                   1e-6 * sum_abs_gx + 1e-7, "dweight vs fp64")
     return dict(dx=ok.mean(), dw=strict_ok(out["dw"], dw).mean(),
                 db=strict_ok(out["db"], db).mean())
+
+
+def device_time(fn):
+    """Milliseconds of device time per call of fn(): the shortest of five runs of four calls."""
+    import torch
+
+    first, last = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    fn()
+    times = []
+    for _ in range(5):
+        first.record()
+        for _ in range(4):
+            fn()
+        last.record()
+        last.synchronize()
+        times.append(first.elapsed_time(last) / 4)
+    return min(times)
