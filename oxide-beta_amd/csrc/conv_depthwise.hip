@@ -10,12 +10,14 @@
 // Sums keep the CPU path's order (bias, then taps by row and column; the input gradient by output
 // row and column), one multiplication and one addition per tap: bit-identical.  An input outside
 // the plane is a +0 operand in place of a skipped tap: the same sum while the weights are finite
-// and the sum does not start at -0.  A tile that starts at -0 or holds a sum that is not finite is
-// taken again tap by tap, the taps outside skipped.
+// and the sum does not start at -0.  A tile at the plane's edge is taken again where they are not
+// or where it does, with -0, which no sum notices, in place of the products outside.
 //
 // The weight gradient gives a channel one block; each thread reads four outputs' gradients and
 // the rows of inputs under them and keeps one sum per tap, by fused multiply-adds.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "conv_mfma.h"
 
@@ -66,13 +68,11 @@ __device__ __forceinline__ void column_masks(int ix, uint32_t W, bool (&mask)[N]
   for (int i = 0; i < N; ++i) mask[i] = static_cast<uint32_t>(ix + i) < W;
 }
 
-template <int A, int B>
-__device__ __forceinline__ bool not_finite(const float (&v)[A][B]) {
+template <int N>
+__device__ __forceinline__ bool not_finite(const float (&v)[N]) {
   float z = 0.0f;
 #pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int j = 0; j < B; ++j) z = __builtin_fmaf(v[i][j], 0.0f, z);
+  for (int i = 0; i < N; ++i) z = __builtin_fmaf(v[i], 0.0f, z);
   return !(z == 0.0f);
 }
 
@@ -87,18 +87,6 @@ __device__ __forceinline__ void store4(float *y, const float *addend, uint64_t a
     for (uint32_t j = 0; j < 4; ++j)
       if (j < count) y[at + j] = addend != nullptr ? v[j] + addend[at + j] : v[j];
   }
-}
-
-// One output of depthwise_kernel, taps outside the plane skipped.
-template <int K, int S, bool Flip>
-__device__ __attribute__((noinline)) float depthwise_one(const float *xp, const float *w, float b,
-                                                         uint32_t H, uint32_t W, int iy, int ix) {
-  for (int t = 0; t < K * K; ++t) {
-    const int y = iy + t / K, x = ix + t % K;
-    if (static_cast<uint32_t>(y) < H && static_cast<uint32_t>(x) < W)
-      b += xp[y * static_cast<int>(W) + x] * w[Flip ? K * K - 1 - t : t];
-  }
-  return b;
 }
 
 // Forward, and (Flip) the input gradient of a stride-1 convolution: source = the output's
@@ -119,41 +107,46 @@ __global__ __launch_bounds__(256, 4) void depthwise_kernel(DepthArgs a) {
 #pragma unroll
   for (int t = 0; t < T; ++t) w[t] = a.w[c * T + t];
   const float b = a.bias != nullptr ? a.bias[c] : 0.0f;
-  bool mask[4 * Q];
-  column_masks(ix0, a.W, mask);
   float acc[TY][TX];
+  auto sum = [&](auto skip, int y0, int x0) {  // Skip: products outside the plane are -0
+    bool mask[4 * Q];
+    column_masks(x0, a.W, mask);
 #pragma unroll
-  for (int i = 0; i < TY; ++i)
+    for (int i = 0; i < TY; ++i)
 #pragma unroll
-    for (int j = 0; j < TX; ++j) acc[i][j] = b;
+      for (int j = 0; j < TX; ++j) acc[i][j] = b;
 #pragma unroll
-  for (int r = 0; r < RY; ++r) {
-    const int iy = iy0 + r;
-    const bool in = static_cast<uint32_t>(iy) < a.H;
-    float row[4 * Q];
-    load_row<Q>(a.x, a.last, static_cast<int>(first + (in ? iy : 0) * a.W) + ix0, in, mask, row);
+    for (int r = 0; r < RY; ++r) {
+      const int iy = y0 + r;
+      const bool in = static_cast<uint32_t>(iy) < a.H;
+      float row[4 * Q];
+      load_row<Q>(a.x, a.last, static_cast<int>(first + (in ? iy : 0) * a.W) + x0, in, mask, row);
 #pragma unroll
-    for (int i = 0; i < TY; ++i) {
-      const int ky = r - i * S;
-      if (ky < 0 || ky >= K) continue;
+      for (int i = 0; i < TY; ++i) {
+        const int ky = r - i * S;
+        if (ky < 0 || ky >= K) continue;
 #pragma unroll
-      for (int kx = 0; kx < K; ++kx)
+        for (int kx = 0; kx < K; ++kx)
 #pragma unroll
-        for (int j = 0; j < TX; ++j)
-          acc[i][j] += row[j * S + kx] * w[Flip ? T - 1 - (ky * K + kx) : ky * K + kx];
+          for (int j = 0; j < TX; ++j) {
+            const float p = row[j * S + kx] * w[Flip ? T - 1 - (ky * K + kx) : ky * K + kx];
+            acc[i][j] += !decltype(skip)::value || (in && mask[j * S + kx]) ? p : -0.0f;
+          }
+      }
     }
+  };
+  sum(std::false_type{}, iy0, ix0);
+  const bool inside = iy0 >= 0 && ix0 >= 0 && iy0 + RY <= static_cast<int>(a.H) &&
+                      ix0 + (TX - 1) * S + K <= static_cast<int>(a.W);
+  if (!inside && (not_finite(w) || __float_as_uint(b) == 0x80000000u)) {
+    int y0 = iy0, x0 = ix0;
+    asm volatile("" : "+v"(y0), "+v"(x0));  // loaded again, not held in registers
+    sum(std::true_type{}, y0, x0);
   }
-  const bool again = not_finite(acc) || __float_as_uint(b) == 0x80000000u;
   const uint64_t out = static_cast<uint64_t>(plane) * a.OH * a.OW;
 #pragma unroll
   for (int i = 0; i < TY; ++i) {
     if (oy0 + i >= a.OH) break;
-    if (again) {
-#pragma unroll
-      for (int j = 0; j < TX; ++j)
-        acc[i][j] = depthwise_one<K, S, Flip>(a.x + first, a.w + c * T, b, a.H, a.W, iy0 + i * S,
-                                              ix0 + j * S);
-    }
     store4(a.y, a.addend, out + (oy0 + i) * a.OW + ox0, a.OW - ox0, acc[i]);
   }
 }
@@ -162,18 +155,6 @@ __global__ __launch_bounds__(256, 4) void depthwise_kernel(DepthArgs a) {
 // oy = a - i through ky = py + 2 i.  A thread: a in {a0, a0 + 1}, b in {b0, b0 + 1}, so 4 x 4
 // inputs under (M2 + 1) x (M2 + 1) outputs, M2 = ceil(K / 2).  x: the gradient (H x W), y: the
 // input's (OH x OW).
-template <int K>
-__device__ __attribute__((noinline)) float depthwise_s2_one(const float *gp, const float *w,
-                                                            uint32_t H, uint32_t W, int y, int x) {
-  float v = 0.0f;  // y, x: with the padding added; output rows ascending
-  for (int ky = K - 1 - ((K - 1 - y) & 1); ky >= 0; ky -= 2)
-    for (int kx = K - 1 - ((K - 1 - x) & 1); kx >= 0; kx -= 2) {
-      const int oy = (y - ky) / 2, ox = (x - kx) / 2;
-      if (y >= ky && x >= kx && static_cast<uint32_t>(oy) < H && static_cast<uint32_t>(ox) < W)
-        v += gp[oy * static_cast<int>(W) + ox] * w[ky * K + kx];
-    }
-  return v;
-}
 template <int K>
 __global__ __launch_bounds__(256, 4) void depthwise_input_s2_kernel(DepthArgs a, uint32_t start) {
   constexpr int T = K * K, M2 = (K + 1) / 2, R = M2 + 1;
@@ -184,49 +165,53 @@ __global__ __launch_bounds__(256, 4) void depthwise_input_s2_kernel(DepthArgs a,
   const uint32_t c = plane - fast_div(plane, a.c_div) * a.C;
   const int a0 = static_cast<int>(start + 2 * ty), b0 = static_cast<int>(start + 2 * tx);
   const uint32_t first = plane * a.H * a.W;
-  float rows[R][4], w[T];  // rows[r][q]: output (a0 - (M2 - 1) + r, b0 - (M2 - 1) + q)
+  float w[T], acc[4][4];
 #pragma unroll
   for (int t = 0; t < T; ++t) w[t] = a.w[c * T + t];
-  bool mask[4];
-  column_masks(b0 - (M2 - 1), a.W, mask);
+  auto sum = [&](auto skip, int oy0, int ox0) {  // as in depthwise_kernel
+    float rows[R][4];  // rows[r][q]: output (oy0 + r, ox0 + q)
+    bool mask[4], in[R];
+    column_masks(ox0, a.W, mask);
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int oy = a0 - (M2 - 1) + r;
-    const bool in = static_cast<uint32_t>(oy) < a.H;
-    load_row<1>(a.x, a.last, static_cast<int>(first + (in ? oy : 0) * a.W) + b0 - (M2 - 1), in,
-                mask, rows[r]);
-  }
-  float acc[4][4];
-#pragma unroll
-  for (int ry = 0; ry < 4; ++ry)
-#pragma unroll
-    for (int rx = 0; rx < 4; ++rx) {
-      float v = 0.0f;
-#pragma unroll
-      for (int i = M2 - 1; i >= 0; --i) {  // oy ascending
-        const int ky = ry % 2 + 2 * i;
-        if (ky >= K) continue;
-#pragma unroll
-        for (int j = M2 - 1; j >= 0; --j) {
-          const int kx = rx % 2 + 2 * j;
-          if (kx < K) v += rows[ry / 2 - i + M2 - 1][rx / 2 - j + M2 - 1] * w[ky * K + kx];
-        }
-      }
-      acc[ry][rx] = v;
+    for (int r = 0; r < R; ++r) {
+      in[r] = static_cast<uint32_t>(oy0 + r) < a.H;
+      load_row<1>(a.x, a.last, static_cast<int>(first + (in[r] ? oy0 + r : 0) * a.W) + ox0, in[r],
+                  mask, rows[r]);
     }
-  const bool again = not_finite(acc);
+#pragma unroll
+    for (int ry = 0; ry < 4; ++ry)
+#pragma unroll
+      for (int rx = 0; rx < 4; ++rx) {
+        float v = 0.0f;
+#pragma unroll
+        for (int i = M2 - 1; i >= 0; --i) {  // oy ascending
+          const int ky = ry % 2 + 2 * i;
+          if (ky >= K) continue;
+#pragma unroll
+          for (int j = M2 - 1; j >= 0; --j) {
+            const int kx = rx % 2 + 2 * j, r = ry / 2 - i + M2 - 1, q = rx / 2 - j + M2 - 1;
+            if (kx >= K) continue;
+            const float p = rows[r][q] * w[ky * K + kx];
+            v += !decltype(skip)::value || (in[r] && mask[q]) ? p : -0.0f;
+          }
+        }
+        acc[ry][rx] = v;
+      }
+  };
+  int oy0 = a0 - (M2 - 1), ox0 = b0 - (M2 - 1);
+  sum(std::false_type{}, oy0, ox0);
+  const bool inside = oy0 >= 0 && ox0 >= 0 && a0 + 1 < static_cast<int>(a.H) &&
+                      b0 + 1 < static_cast<int>(a.W);
+  if (!inside && not_finite(w)) {
+    asm volatile("" : "+v"(oy0), "+v"(ox0));
+    sum(std::true_type{}, oy0, ox0);
+  }
   const int x0 = 2 * b0 - a.pad;  // -1 where the padding is odd
   const uint64_t out = static_cast<uint64_t>(plane) * a.OH * a.OW;
 #pragma unroll
   for (int ry = 0; ry < 4; ++ry) {
     const int y = 2 * a0 + ry - a.pad;
     if (static_cast<uint32_t>(y) >= a.OH) continue;
-    if (again) {
-#pragma unroll
-      for (int rx = 0; rx < 4; ++rx)
-        acc[ry][rx] = depthwise_s2_one<K>(a.x + first, a.w + c * T, a.H, a.W, 2 * a0 + ry,
-                                          2 * b0 + rx);
-    }
     const uint64_t at = out + static_cast<uint32_t>(y) * a.OW;
     if (x0 >= 0) {
       if (static_cast<uint32_t>(x0) < a.OW) store4(a.y, a.addend, at + x0, a.OW - x0, acc[ry]);
@@ -241,13 +226,13 @@ __global__ __launch_bounds__(256, 4) void depthwise_input_s2_kernel(DepthArgs a,
   }
 }
 
-// Weight gradient: block per channel and chunk of images; a thread item is a TY x 4 tile of outputs,
-// whose products go to one sum per tap by fused multiply-adds; wave sums in a fixed order, waves in
-// order.  Operands outside are +0; a thread that ends with a sum that is not finite walks its items
+// Weight gradient: block per channel and chunk of images; a thread item is a TY x 4 tile of
+// outputs, whose products go to one sum per tap by fused multiply-adds; wave sums in a fixed order,
+// waves in order.  Operands outside are +0; a thread that ends with a sum that is not finite walks its items
 // again, skipping them.  Bound by the loads a CU issues: the tile shares each row of inputs among
 // its outputs' rows.  64 images of 192 x 28 x 28, 5 x 5: 157 -> 29 us; 32 of 64 x 28 x 28, 5 x 5:
-// 51 -> 14.5 us; 32 of 32 x 112 x 112, 3 x 3: 305 -> 29 us.  5 x 5 kernels take three waves per
-// SIMD (at four their rows spill: 14 against 18 us for 192 x 28 x 28 at stride 2).
+// 51 -> 14.5 us; 32 of 32 x 112 x 112, 3 x 3: 305 -> 29 us.  5 x 5 kernels are bound to three waves
+// per SIMD (bound to four, their rows spilled: 14 against 18 us for 192 x 28 x 28 at stride 2).
 struct DepthWeightArgs {
   const float *g, *x;
   float *dw;
@@ -255,81 +240,63 @@ struct DepthWeightArgs {
   int pad, g_last, x_last;
   FastDiv tiles_x_div, tiles_y_div;
 };
-template <int K, int S, int TY, int Threads>
-__device__ __attribute__((noinline)) float depthwise_weight_one(const DepthWeightArgs &a,
-                                                                uint32_t c, uint32_t begin,
-                                                                uint32_t end, int t) {
-  float acc = 0.0f;
-  for (uint32_t item = begin + threadIdx.x; item < end; item += Threads) {
-    const uint32_t t0 = fast_div(item, a.tiles_x_div), ox0 = 4 * (item - t0 * a.tiles_x);
-    const uint32_t n = fast_div(t0, a.tiles_y_div), oy0 = TY * (t0 - n * a.tiles_y);
-    const uint32_t plane = n * a.C + c;
-    for (uint32_t oy = oy0; oy < oy0 + TY && oy < a.OH; ++oy) {
-      const int iy = static_cast<int>(oy * S) - a.pad + t / K;
-      if (static_cast<uint32_t>(iy) >= a.H) continue;
-      for (uint32_t ox = ox0; ox < ox0 + 4 && ox < a.OW; ++ox) {
-        const int ix = static_cast<int>(ox * S) - a.pad + t % K;
-        if (static_cast<uint32_t>(ix) < a.W)
-          acc = __builtin_fmaf(a.g[(plane * a.OH + oy) * a.OW + ox],
-                               a.x[(plane * a.H + iy) * a.W + ix], acc);
-      }
-    }
-  }
-  return acc;
-}
 template <int K, int S, int Threads>
-__global__ __launch_bounds__(Threads, K == 5 ? 3 : 4) void depthwise_weight_kernel(DepthWeightArgs a) {
+__global__ __launch_bounds__(Threads, K == 5 ? 3 : 4) void depthwise_weight_kernel(
+    DepthWeightArgs a) {
   constexpr int T = K * K, Q = (3 * S + K + 3) / 4, TY = S == 1 ? 4 : 2, RY = (TY - 1) * S + K;
   __shared__ float sums[Threads / 64][T];
   const uint32_t c = blockIdx.x, begin = blockIdx.y * a.per_chunk;
   const uint32_t end = begin + a.per_chunk < a.items ? begin + a.per_chunk : a.items;
-  float acc[1][T];
+  float acc[T];
+  auto walk = [&](auto skip) {  // Skip: products outside either plane are left out
 #pragma unroll
-  for (int t = 0; t < T; ++t) acc[0][t] = 0.0f;
-  for (uint32_t item = begin + threadIdx.x; item < end; item += Threads) {
-    const uint32_t t0 = fast_div(item, a.tiles_x_div), ox0 = 4 * (item - t0 * a.tiles_x);
-    const uint32_t n = fast_div(t0, a.tiles_y_div), oy0 = TY * (t0 - n * a.tiles_y);
-    const uint32_t plane = n * a.C + c;
-    const int iy0 = static_cast<int>(oy0 * S) - a.pad, ix0 = static_cast<int>(ox0 * S) - a.pad;
-    float gv[TY][4];
-    bool gmask[4], mask[4 * Q];
-    column_masks(static_cast<int>(ox0), a.OW, gmask);
-    column_masks(ix0, a.W, mask);
-#pragma unroll
-    for (int i = 0; i < TY; ++i) {
-      const bool in = oy0 + i < a.OH;
-      load_row<1>(a.g, a.g_last,
-                  static_cast<int>((plane * a.OH + (in ? oy0 + i : 0)) * a.OW + ox0), in, gmask,
-                  gv[i]);
-    }
-#pragma unroll
-    for (int r = 0; r < RY; ++r) {
-      const int iy = iy0 + r;
-      const bool in = static_cast<uint32_t>(iy) < a.H;
-      float row[4 * Q];
-      load_row<Q>(a.x, a.x_last, static_cast<int>((plane * a.H + (in ? iy : 0)) * a.W) + ix0, in,
-                  mask, row);
+    for (int t = 0; t < T; ++t) acc[t] = 0.0f;
+    for (uint32_t item = begin + threadIdx.x; item < end; item += Threads) {
+      const uint32_t t0 = fast_div(item, a.tiles_x_div), ox0 = 4 * (item - t0 * a.tiles_x);
+      const uint32_t n = fast_div(t0, a.tiles_y_div), oy0 = TY * (t0 - n * a.tiles_y);
+      const uint32_t plane = n * a.C + c;
+      const int iy0 = static_cast<int>(oy0 * S) - a.pad, ix0 = static_cast<int>(ox0 * S) - a.pad;
+      float gv[TY][4];
+      bool gmask[4], mask[4 * Q];
+      column_masks(static_cast<int>(ox0), a.OW, gmask);
+      column_masks(ix0, a.W, mask);
 #pragma unroll
       for (int i = 0; i < TY; ++i) {
-        const int ky = r - i * S;
-        if (ky < 0 || ky >= K) continue;
+        const bool in = oy0 + i < a.OH;
+        load_row<1>(a.g, a.g_last,
+                    static_cast<int>((plane * a.OH + (in ? oy0 + i : 0)) * a.OW + ox0), in, gmask,
+                    gv[i]);
+      }
 #pragma unroll
-        for (int kx = 0; kx < K; ++kx)
+      for (int r = 0; r < RY; ++r) {
+        const int iy = iy0 + r;
+        const bool in = static_cast<uint32_t>(iy) < a.H;
+        float row[4 * Q];
+        load_row<Q>(a.x, a.x_last, static_cast<int>((plane * a.H + (in ? iy : 0)) * a.W) + ix0, in,
+                    mask, row);
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            acc[0][ky * K + kx] = __builtin_fmaf(gv[i][j], row[j * S + kx], acc[0][ky * K + kx]);
+        for (int i = 0; i < TY; ++i) {
+          const int ky = r - i * S;
+          if (ky < 0 || ky >= K) continue;
+#pragma unroll
+          for (int kx = 0; kx < K; ++kx)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int t = ky * K + kx;
+              const float v = __builtin_fmaf(gv[i][j], row[j * S + kx], acc[t]);
+              const bool at = oy0 + i < a.OH && gmask[j] && in && mask[j * S + kx];
+              acc[t] = !decltype(skip)::value || at ? v : acc[t];
+            }
+        }
       }
     }
-  }
-  if (not_finite(acc)) {
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-      acc[0][t] = depthwise_weight_one<K, S, TY, Threads>(a, c, begin, end, t);
-  }
-  wave_sums_rows(acc[0]);
+  };
+  walk(std::false_type{});
+  if (not_finite(acc)) walk(std::true_type{});
+  wave_sums_rows(acc);
   if (threadIdx.x % 64 == 0) {
 #pragma unroll
-    for (int t = 0; t < T; ++t) sums[threadIdx.x / 64][t] = acc[0][t];
+    for (int t = 0; t < T; ++t) sums[threadIdx.x / 64][t] = acc[t];
   }
   __syncthreads();
   if (threadIdx.x < T) {
@@ -372,7 +339,8 @@ WeightSplit weight_split(const Dims &d) {
 template <int Threads>
 void launch_weight(hipStream_t s, const Dims &d, const DepthWeightArgs &a, uint32_t chunks) {
   const dim3 grid(d.in_c, chunks), block(Threads);
-  if (d.k == 3 && d.stride == 1) launch(depthwise_weight_kernel<3, 1, Threads>, grid, block, 0, s, a);
+  if (d.k == 3 && d.stride == 1)
+    launch(depthwise_weight_kernel<3, 1, Threads>, grid, block, 0, s, a);
   else if (d.k == 3) launch(depthwise_weight_kernel<3, 2, Threads>, grid, block, 0, s, a);
   else if (d.stride == 1) launch(depthwise_weight_kernel<5, 1, Threads>, grid, block, 0, s, a);
   else launch(depthwise_weight_kernel<5, 2, Threads>, grid, block, 0, s, a);
