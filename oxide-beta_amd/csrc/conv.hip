@@ -38,6 +38,8 @@
 //     weight-chunk) element per thread.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <string>
 #include <type_traits>
 
@@ -2709,28 +2711,70 @@ MfmaWeightPlan weight_mfma_plan(const ConvGeom &g, bool bias = false) {
 }
 
 // Ungrouped square convolutions run on the matrix cores over flattened positions (conv_mfma.h)
-// where no per-image LDS kernel takes them, and where one does but the layer has over 2^27
-// products: a block per image and channel tile then restages its planes for every tile (64
-// images of 64 x 14 x 14 to 64 channels, 3 x 3: 51 against 24 us forward, 57 against 24 us input
-// gradient; 16 images, 2^26.8 products: 23 us both ways; the 128-image 7 x 7 to 96-channel
-// stride-2 layer, 2^25.8: 9 against 14 us, so smaller layers keep the per-image kernels).  A
-// stride-2 input gradient has a quarter of the blocks: twice that (14 x 14 to 128 channels: 64
-// images, 2^27.8: 35 against 42 us; 128 images: 68 against 43 us).
+// where a per-image LDS kernel takes them but the layer has over 2^27 products: a block per image
+// and channel tile then restages its planes for every tile (64 images of 64 x 14 x 14 to 64
+// channels, 3 x 3: 51 against 24 us forward, 57 against 24 us input gradient; 16 images, 2^26.8
+// products: 23 us both ways; the 128-image 7 x 7 to 96-channel stride-2 layer, 2^25.8: 9 against 14
+// us, so smaller layers keep the per-image kernels).  A stride-2 input gradient has a quarter of
+// the blocks: twice that (14 x 14 to 128 channels: 64 images, 2^27.8: 35 against 42 us; 128
+// images: 68 against 43 us).  Few rows of a 32-row tile keep the per-image kernels too, whose tile
+// is four channels: up to four (1024 images of 64 x 14 x 14 to 4: 53 against 81 us; to 6: 110
+// against 80), up to eight where the reduced channels are 16 and fewer (1024 of 16 x 16 x 16 to 8,
+// 5 x 5: 63 against 88 us), and up to 16 in a stride-2 input gradient.
 constexpr uint64_t kLargeProducts = 1ull << 27;
 uint64_t products(const ConvGeom &g) {
   return static_cast<uint64_t>(g.batch) * g.oh * g.ow * g.out_c * g.in_per_group * g.kh * g.kw;
 }
+// Where no per-image kernel takes them, the rule is an estimate of both kernels' times in us, in
+// terms per sum (reduced channels x taps) times the larger of a chain's pace and the chip's rate.
+// The kernel of one output per thread: 0.026 us a term (0.036 where its loads are strided) while
+// its outputs fill the chip once, 0.045 over 80 000 outputs (a second wave per SIMD), then 2.6e-7
+// us a product (6e-7 strided).  The matrix cores: 0.029 us a term along a wave's chain, 3.1e-8 us a
+// product of whole 32-row tiles, 4 us more to start.  So they lose layers that leave the chip idle
+// (1 image of 64 x 28 x 28 to 64, 3 x 3: 14 against 22 us; 2 of 512 x 7 x 7 to 512, stride 2, input
+// gradient: 110 against 144) and layers of one to three rows (32 images of 64 x 112 x 112 to 1,
+// 3 x 3: 68 against 148 us; to 2: 116 against 149; to 4: 215 against 149).
+struct PairTime {
+  double threads, tiles;
+};
+PairTime square_times(const ConvGeom &g, bool forward) {
+  const double taps = static_cast<double>(g.kh) * g.kw;
+  const double c = forward ? g.in_c : g.out_c, m = forward ? g.out_c : g.in_c;
+  const double n = static_cast<double>(g.batch) * (forward ? g.oh * g.ow : g.h * g.w);
+  const double outputs = n * m, padded = n * std::ceil(m / 32) * 32;
+  const double terms = c * taps, paired = std::ceil(c / 2) * 2 * taps;  // tiles: channel pairs
+  const bool strided = g.stride > 1, phases = strided && !forward;  // of a stride-2 gradient
+  if (taps == 1) {  // a strided or padded 1 x 1: cache lines of one value each
+    const double tile = phases ? std::max(0.045, 1e-8 * padded) : std::max(0.06, 3.1e-8 * padded);
+    return {terms * std::max(0.2, (phases ? 8e-7 : 1e-6) * outputs),
+            (phases ? 2.5 : 1.3) + paired * tile};
+  }
+  if (phases)  // a quarter of the terms per input
+    return {terms * std::max(0.018, 2e-7 * outputs), 4 + paired * std::max(0.029, 1e-8 * padded)};
+  const double tiles = 4 + paired * std::max(0.029, 3.1e-8 * padded);
+  if (strided)
+    return {terms * std::max(outputs < 2048 ? 0.018 : 0.036, 6e-7 * outputs), tiles};
+  return {terms * std::max(outputs > 80e3 ? 0.045 : 0.026, 2.6e-7 * outputs), tiles};
+}
+bool tiles_pay(const ConvGeom &g, bool forward) {
+  const PairTime t = square_times(g, forward);
+  return t.tiles < t.threads;
+}
 bool large_forward(const ConvGeom &g) {
-  return g.groups == 1 && g.kh == g.kw &&
-         (products(g) > kLargeProducts ||
-          (forward_lds_plan(g).tile == 0 && forward_split_plan(g).tile == 0)) &&
+  if (g.groups != 1 || g.kh != g.kw) return false;
+  const bool per_image = forward_lds_plan(g).tile > 0 || forward_split_plan(g).tile > 0;
+  return (per_image ? products(g) > kLargeProducts && g.out_c > (g.in_c <= 16 ? 8u : 4u)
+                    : tiles_pay(g, true)) &&
          oxh::conv_mfma::takes_forward(mfma_dims(g));
 }
 bool large_input_backward(const ConvGeom &g) {
-  return g.groups == 1 && g.kh == g.kw &&
-         (products(g) > g.stride * kLargeProducts ||
-          (input_backward_mfma_plan(g).lds_bytes == 0 &&
-           input_backward_s2_plan(g).lds_bytes == 0 && input_backward_lds_plan(g).tile == 0)) &&
+  if (g.groups != 1 || g.kh != g.kw) return false;
+  const bool per_image = input_backward_mfma_plan(g).lds_bytes > 0 ||
+                         input_backward_s2_plan(g).lds_bytes > 0 ||
+                         input_backward_lds_plan(g).tile > 0;
+  const uint32_t rows = g.stride > 1 ? 16 : g.out_c <= 16 ? 8 : 4;
+  return (per_image ? products(g) > g.stride * kLargeProducts && g.in_c > rows
+                    : tiles_pay(g, false)) &&
          oxh::conv_mfma::takes_input_backward(mfma_dims(g));
 }
 

@@ -17,16 +17,16 @@ pytestmark = pytest.mark.gpu
 
 # batch, in, height, width, out, kernel, stride, padding
 CASES = [
-    (1, 3, 75, 73, 33, 3, 2, 1),      # a stem: one and a half channel pairs, 33 output rows
-    (2, 32, 33, 31, 32, 3, 1, 1),     # one row tile, odd planes, positions across images
-    (3, 17, 40, 29, 70, 3, 1, 1),     # an odd channel, 64 + 6 rows
+    (40, 3, 75, 73, 33, 3, 2, 1),     # a stem: one and a half channel pairs, 33 output rows
+    (6, 32, 33, 31, 32, 3, 1, 1),     # one row tile, odd planes, positions across images
+    (6, 17, 40, 29, 70, 3, 1, 1),     # an odd channel, 64 + 6 rows
     (1, 64, 65, 66, 64, 3, 1, 1),     # whole tiles
-    (2, 40, 30, 34, 96, 3, 2, 1),
-    (2, 24, 41, 37, 40, 5, 1, 2),
-    (1, 10, 61, 43, 24, 5, 2, 2),
+    (8, 40, 30, 34, 96, 3, 2, 1),
+    (4, 24, 41, 37, 40, 5, 1, 2),
+    (12, 10, 61, 43, 24, 5, 2, 2),
     (2, 96, 32, 31, 64, 1, 2, 0),     # a strided 1 x 1: three of four inputs feed no output
-    (2, 20, 33, 33, 20, 3, 1, 0),     # no padding
-    (1, 70, 35, 20, 16, 3, 2, 0),
+    (14, 20, 33, 33, 20, 3, 1, 0),    # no padding
+    (16, 70, 35, 20, 16, 3, 2, 0),
     (1, 24, 35, 33, 20, 1, 1, 1),     # a padded 1 x 1
     (20, 48, 17, 16, 66, 3, 1, 1),    # planes a per-image kernel holds, over 2^27 products
     (60, 64, 15, 14, 144, 3, 2, 1),
@@ -73,7 +73,7 @@ def test_input_gradient(module, dev, case, addend):
 
 
 @pytest.mark.parametrize("value", [np.inf, np.nan])
-@pytest.mark.parametrize("case", [(2, 33, 34, 31, 40, 3, 1, 1), (1, 30, 40, 44, 66, 3, 2, 1)])
+@pytest.mark.parametrize("case", [(8, 33, 34, 31, 40, 3, 1, 1), (8, 30, 40, 44, 66, 3, 2, 1)])
 def test_weights_that_are_not_finite(module, dev, case, value):
     """An infinite or NaN weight reaches the outputs whose tap lies inside the input, and no
     other: taps outside are skipped, as the CPU path skips them."""
@@ -117,7 +117,7 @@ def test_weight_gradient(module, dev, case):
 
 
 @pytest.mark.parametrize("value", [np.inf, np.nan])
-@pytest.mark.parametrize("case", [(2, 33, 34, 31, 40, 3, 1, 1), (1, 30, 40, 44, 66, 3, 2, 1)])
+@pytest.mark.parametrize("case", [(8, 33, 34, 31, 40, 3, 1, 1), (8, 30, 40, 44, 66, 3, 2, 1)])
 def test_gradients_that_are_not_finite(module, dev, case, value):
     """An infinite or NaN output gradient in a corner reaches the weights whose tap lies inside
     the input there, and no other."""
