@@ -2905,12 +2905,23 @@ int input_splits(const ProductArgs &x) {
 // Pointwise forwards and input gradients on the matrix cores (conv_pointwise_mfma.hip): layers of
 // over 2^27 products, and planes of over 64 positions but for the small grids of many channels
 // that the split tiles take (8 images of 960 x 9 x 9 to 33 channels: 8.6 us, against 15 us for the
-// channel split there).  Smaller layers keep the CPU path's order.
+// channel split there) and for small layers, which end before a wave there has its chunks of
+// channels in flight: under 2^22.6 products and 800 000 values read and written (1 image of 128 x
+// 14 x 14 to 128: 4.1 against 5.2 us; 4 of 64 x 28 x 28 to 64: 5.8 against 4.6).  An input gradient
+// shares its launch with the weight gradient in a whole backward, so its line is later, 2^25
+// products and 1 200 000 values (4 images of 64 x 28 x 28 to 64: 11 us in one launch, 18 us in
+// several; 4 of 64 x 56 x 56: 20 against 18), or 100 000 positions of a few channels (79 images of
+// 4 x 44 x 44 to 1: 30 against 23 us).  Smaller layers keep the CPU path's order.
 bool large_pointwise(const ConvGeom &g, bool forward) {
   if (!pointwise(g)) return false;
   const uint32_t plane = g.h * g.w, m = forward ? g.out_c : g.in_c, k = forward ? g.in_c : g.out_c;
-  return ((products(g) > kLargeProducts && plane >= 16) ||
-          (plane > 64 && split_kind(m, g.batch * plane, k, 1) == 0)) &&
+  const uint64_t positions = static_cast<uint64_t>(g.batch) * plane;
+  const uint64_t values = positions * (static_cast<uint64_t>(k) + m), count = products(g);
+  const bool enough = forward ? count >= 6350000 || values >= 800000 ||
+                                    (positions >= 100000 && k > 1)
+                              : count >= (1u << 25) || values >= 1200000 || positions >= 100000;
+  return ((count > kLargeProducts && plane >= 16) ||
+          (plane > 64 && enough && split_kind(m, g.batch * plane, k, 1) == 0)) &&
          oxh::conv_mfma::takes_pointwise(g.batch, plane, k, m);
 }
 

@@ -47,3 +47,18 @@ def test_forward(case, serial):
 ])
 def test_input_gradient(case, serial):
     assert _serial(*case, forward=False) == serial
+
+
+# 1 x 1 layers: batch, in, height, width, out
+@pytest.mark.parametrize("case,forward,backward", [
+    ((1, 128, 14, 14, 128), True, True),         # a few waves' worth of products
+    ((1, 32, 64, 64, 16), True, True),
+    ((4, 64, 28, 28, 64), False, True),          # a backward whose gradients share a launch
+    ((1, 64, 56, 56, 64), False, True),
+    ((79, 4, 44, 44, 1), False, False),          # few channels, many positions
+    ((8, 64, 56, 56, 64), False, False),
+    ((64, 64, 56, 56, 192), False, False),
+])
+def test_pointwise(case, forward, backward):
+    assert _serial(*case, 1, 1, 0, forward=True) == forward
+    assert _serial(*case, 1, 1, 0, forward=False) == backward

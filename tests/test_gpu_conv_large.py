@@ -228,8 +228,8 @@ def test_paired_backward_leaves_wide_bias_sums_to_their_kernel(module, dev):
 # CU), single ones (odd planes; few blocks), four waves per position; ragged rows, positions
 # and channel chunks (16, 32 and 128 channels); a plane of 64 in a layer of over 2^27 products
 POINTWISE = [
-    (15, 37, 60, 150, 33), (16, 40, 93, 91, 70), (5, 33, 31, 13, 50), (3, 129, 11, 9, 40),
-    (1, 70, 9, 9, 5), (1, 200, 13, 6, 96), (6, 400, 10, 8, 130), (40, 130, 8, 8, 416),
+    (15, 37, 60, 150, 33), (16, 40, 93, 91, 70), (36, 33, 31, 13, 50), (66, 129, 11, 9, 40),
+    (200, 70, 9, 9, 5), (23, 200, 13, 6, 96), (9, 400, 10, 8, 130), (40, 130, 8, 8, 416),
 ]
 
 
