@@ -1445,9 +1445,8 @@ __global__ __launch_bounds__(256) void conv2d_bias_kernel(BiasArgs a) { bias_blo
 // images of 64 x 56 x 56 took 131 us and now 8 us; 32 of 32 x 112 x 112, 547 us and now 22 us (32
 // blocks: bound by what one CU loads).  A channel's terms have to meet in one block, as the entry
 // point has no workspace.  The line is where a wave's dependent rounds of loads (6272 terms: 13 us
-// on the device) outlast the block's barrier and sums (4 us).  The paired 1 x 1 launch carries the
-// bias sums up to this many terms only, a wave per channel.
-constexpr uint32_t kWideBias = 4096;
+// on the device) outlast the block's barrier and sums (4 us).
+constexpr uint32_t kWideBias = 4096, kPairedBias = 7168;
 constexpr int kWideBiasThreads = 1024;
 template <bool Vec>
 __global__ __launch_bounds__(kWideBiasThreads) void conv2d_wide_bias_kernel(BiasArgs a) {
@@ -1485,9 +1484,6 @@ __global__ __launch_bounds__(kWideBiasThreads) void conv2d_wide_bias_kernel(Bias
   a.out[oc] = sum;
 }
 uint32_t bias_blocks(uint32_t out_c) { return (out_c + 3) / 4; }
-bool wide_bias(const ConvGeom &g) {
-  return static_cast<uint64_t>(g.batch) * g.oh * g.ow > kWideBias;
-}
 BiasArgs bias_args(const ConvGeom &g, const float *gradient, float *bias_gradient) {
   return BiasArgs{gradient, bias_gradient, g.batch, g.out_c, g.oh * g.ow,
                   oxh::make_fastdiv(g.oh * g.ow)};
@@ -2923,6 +2919,15 @@ bool large_pointwise(const ConvGeom &g, bool forward) {
   return ((count > kLargeProducts && plane >= 16) ||
           (plane > 64 && enough && split_kind(m, g.batch * plane, k, 1) == 0)) &&
          oxh::conv_mfma::takes_pointwise(g.batch, plane, k, m);
+}
+
+// The bias kernel of a layer.  A 1 x 1 backward in one launch sums the bias in passing, a wave per
+// channel, which outlasts its products only from about 7000 terms on (42 images of 30 x 10 x 10 to 9,
+// 4200 terms: 7.6 us, 10.2 with a launch of its own; 12 000 terms: 0.77 of the time); the bias entry
+// point follows, so that both leave the same bits.
+bool wide_bias(const ConvGeom &g) {
+  const bool paired = pointwise(g) && !large_pointwise(g, false);
+  return static_cast<uint64_t>(g.batch) * g.oh * g.ow > (paired ? kPairedBias : kWideBias);
 }
 
 // One-wave 8 x 8 serial tiles hold ~9.5 KB of LDS each: 16 blocks per CU, 4096 on the chip at

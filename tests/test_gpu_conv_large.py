@@ -211,9 +211,9 @@ def test_paired_backward_leaves_wide_bias_sums_to_their_kernel(module, dev):
     """A 1 x 1 backward whose two products share a launch, with more bias terms than a wave sums:
     the bias equals the separate entry point's, bit for bit."""
     r = np.random.default_rng(5)
-    shape = ox.conv2d_shape(110, 16, 7, 7, 16, 1, 1, 0, 1)
-    x = to_dev(r.standard_normal((110, 16, 7, 7)).astype(np.float32), dev)
-    g = to_dev(r.standard_normal((110, 16, 7, 7)).astype(np.float32), dev)
+    shape = ox.conv2d_shape(150, 16, 7, 7, 16, 1, 1, 0, 1)
+    x = to_dev(r.standard_normal((150, 16, 7, 7)).astype(np.float32), dev)
+    g = to_dev(r.standard_normal((150, 16, 7, 7)).astype(np.float32), dev)
     wt = to_dev(r.standard_normal((16, 16, 1, 1)).astype(np.float32), dev)
     dx, dw = torch.empty_like(x), torch.empty_like(wt)
     db, ref = (torch.full((16,), float("nan"), device=dev) for _ in range(2))
