@@ -2996,16 +2996,34 @@ bool depthwise_single_pass(const ConvGeom &g) {
          (g.kh == 3 || g.kh == 5) && g.out_c <= 65535 * 16;
 }
 
-// Those of them with four and more columns run in tiles (conv_depthwise.hip): as fast at the
-// smallest (8 images of 72 x 4 x 4: 7 to 9 us both ways, the launch) and up to ten times as fast
-// at the largest.  The weight gradient of a 3 x 3 kernel at stride 2 keeps a thread per position up
-// to 64 of them, where half of each tile's loads would be for nothing (32 images of 576 x 14 x 14:
-// 10.1 against 13.4 us; 96 x 56 x 56: 39 against 21 us).
-bool tiled_depthwise(const ConvGeom &g) {
-  return depthwise_single_pass(g) && oxh::conv_mfma::takes_depthwise(mfma_dims(g));
+// Those of them with four and more columns run in tiles (conv_depthwise.hip) from five million
+// products on, 2.8 million in a stride-2 forward: a tile's rows of loads and sums follow each other,
+// 4 to 6 us, which small layers do not hide (2 images of 39 x 10 x 10, 3 x 3: 2.5 against 4.4 us
+// forward and input gradient; at the line both take 4 to 5 us; 64 of 192 x 28 x 28, 5 x 5: 124
+// against 21).  One channel is also an ungrouped layer, whose kernels take as long a chain: tiles
+// from 196 outputs on, and for every input gradient (8 images of 1 x 86 x 86, 5 x 5, stride 2: 174
+// against 4 us).
+bool tiled_depthwise(const ConvGeom &g, bool forward) {
+  if (!depthwise_single_pass(g) || !oxh::conv_mfma::takes_depthwise(mfma_dims(g))) return false;
+  if (g.in_c == 1 && (!forward || g.oh * g.ow > 196)) return true;
+  const uint64_t values = static_cast<uint64_t>(g.batch) * g.in_c *
+                          (forward ? g.oh * g.ow : g.h * g.w);
+  return values * g.kh * g.kw >= (forward && g.stride == 2 ? 2800000u : 5000000u);
 }
+// Their weight gradient, by the outputs of a channel, which one block or a few walk: 3 x 3 from 4000
+// on (stride 2: 2900), 5 x 5 from 2080 (stride 2: 1040), or 1000 where 128 channels and more fill
+// the chip (19 images of 3 x 23 x 23, 3 x 3, stride 2: 3.0 against 4.1 us; 2 of 58 x 50 x 50: 6.2
+// against 6.5; 17 of 293 x 14 x 15, 5 x 5: 15 against 8).  A 3 x 3 kernel at stride 2 keeps a thread
+// per position up to 64 of a plane, where half of each tile's loads would be for nothing (32 images
+// of 576 x 14 x 14: 10.1 against 13.4 us; 96 x 56 x 56: 39 against 21 us), and up to eight columns
+// where the channels fill the chip without chunks (98 of 469 x 99 x 11: 75 against 113 us).
 bool tiled_depthwise_weight(const ConvGeom &g) {
-  return tiled_depthwise(g) && !(g.kh == 3 && g.stride == 2 && g.oh * g.ow <= 64);
+  if (!depthwise_single_pass(g) || !oxh::conv_mfma::takes_depthwise(mfma_dims(g))) return false;
+  const bool strided = g.stride == 2;
+  if (g.kh == 3 && strided && (g.oh * g.ow <= 64 || (g.ow <= 8 && g.in_c >= 256))) return false;
+  const uint64_t outputs = static_cast<uint64_t>(g.batch) * g.oh * g.ow;
+  if (g.kh == 3) return outputs >= (strided ? 2900u : 4000u);
+  return outputs >= (g.in_c >= 128 ? 1000u : strided ? 1040u : 2080u);
 }
 
 // Ungrouped weight gradients the per-image matrix-core kernel (weight_mfma_plan) does not take run
@@ -3255,7 +3273,7 @@ oxh_status input_backward_impl(const char *name, oxh_stream stream,
     const ProductArgs x = input_product(g, gradient, weight, addend, input_gradient);
     return launch_product(name, s, x, 1, input_splits(x) != 0);
   }
-  if (tiled_depthwise(g)) {
+  if (tiled_depthwise(g, false)) {
     oxh::conv_mfma::depthwise_input_backward(s, mfma_dims(g), gradient, weight, addend,
                                              input_gradient);
     return oxh::launched(name);
@@ -3511,7 +3529,7 @@ oxh_status oxh_conv2d_forward(oxh_stream stream, const oxh_conv2d_shape *shape,
     a.k_chunk = a.K;
     return launch_product(name, s, a, 1, true);
   }
-  if (tiled_depthwise(g)) {
+  if (tiled_depthwise(g, true)) {
     oxh::conv_mfma::depthwise_forward(s, mfma_dims(g), input, weight, bias, output);
     return oxh::launched(name);
   }

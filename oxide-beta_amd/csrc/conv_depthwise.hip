@@ -228,9 +228,9 @@ __global__ __launch_bounds__(256, 4) void depthwise_input_s2_kernel(DepthArgs a,
 
 // Weight gradient: block per channel and chunk of images; a thread item is a TY x 4 tile of
 // outputs, whose products go to one sum per tap by fused multiply-adds; wave sums in a fixed order,
-// waves in order.  Operands outside are +0; a thread that ends with a sum that is not finite walks its items
-// again, skipping them.  Bound by the loads a CU issues: the tile shares each row of inputs among
-// its outputs' rows.  64 images of 192 x 28 x 28, 5 x 5: 157 -> 29 us; 32 of 64 x 28 x 28, 5 x 5:
+// waves in order.  Operands outside are +0; a thread that ends with a sum that is not finite walks
+// its items again, skipping them.  Bound by the loads a CU issues: the tile shares each row of
+// inputs among its outputs' rows.  64 images of 192 x 28 x 28, 5 x 5: 157 -> 29 us; 32 of 64 x 28 x 28, 5 x 5:
 // 51 -> 14.5 us; 32 of 32 x 112 x 112, 3 x 3: 305 -> 29 us.  5 x 5 kernels are bound to three waves
 // per SIMD (bound to four, their rows spilled: 14 against 18 us for 192 x 28 x 28 at stride 2).
 struct DepthWeightArgs {
@@ -339,10 +339,14 @@ WeightSplit weight_split(const Dims &d) {
 template <int Threads>
 void launch_weight(hipStream_t s, const Dims &d, const DepthWeightArgs &a, uint32_t chunks) {
   const dim3 grid(d.in_c, chunks), block(Threads);
-  if (d.k == 3 && d.stride == 1)
-    launch(depthwise_weight_kernel<3, 1, Threads>, grid, block, 0, s, a);
-  else if (d.k == 3) launch(depthwise_weight_kernel<3, 2, Threads>, grid, block, 0, s, a);
-  else if (d.stride == 1) launch(depthwise_weight_kernel<5, 1, Threads>, grid, block, 0, s, a);
+  if constexpr (Threads > 64) {  // 3 x 3 layers of so few tiles take another kernel (conv.hip)
+    if (d.k == 3 && d.stride == 1)
+      launch(depthwise_weight_kernel<3, 1, Threads>, grid, block, 0, s, a);
+    else if (d.k == 3)
+      launch(depthwise_weight_kernel<3, 2, Threads>, grid, block, 0, s, a);
+    if (d.k == 3) return;
+  }
+  if (d.stride == 1) launch(depthwise_weight_kernel<5, 1, Threads>, grid, block, 0, s, a);
   else launch(depthwise_weight_kernel<5, 2, Threads>, grid, block, 0, s, a);
 }
 
@@ -408,7 +412,7 @@ void depthwise_weight_backward(hipStream_t s, const Dims &d, const float *gradie
   a.tiles_x = w.tiles_x, a.tiles_y = w.tiles_y, a.items = w.items, a.per_chunk = w.per_chunk;
   a.tiles_x_div = make_fastdiv(w.tiles_x), a.tiles_y_div = make_fastdiv(w.tiles_y);
   // a wave or four where that is about a tile per thread; eight where channels leave CUs idle
-  if (w.items <= 128) launch_weight<64>(s, d, a, w.chunks);
+  if (w.items <= 128 && d.k == 5) launch_weight<64>(s, d, a, w.chunks);
   else if (w.items <= 512 || d.in_c * w.chunks > 256) launch_weight<256>(s, d, a, w.chunks);
   else launch_weight<512>(s, d, a, w.chunks);
 }

@@ -173,3 +173,16 @@ def device_time(fn):
         last.synchronize()
         times.append(first.elapsed_time(last) / 4)
     return min(times)
+
+
+def graph_time(fn, calls=40):
+    """Milliseconds of device time per call of fn() in a replayed graph of `calls` of them."""
+    import torch
+
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        fn()
+    with torch.cuda.graph(graph, stream=stream):
+        for _ in range(calls):
+            fn()
+    return device_time(graph.replay) / calls
