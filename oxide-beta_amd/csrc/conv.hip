@@ -3027,22 +3027,34 @@ bool tiled_depthwise_weight(const ConvGeom &g) {
 }
 
 // Ungrouped weight gradients the per-image matrix-core kernel (weight_mfma_plan) does not take run
-// on the matrix cores over groups of output rows (conv_weight_mfma.hip), but for short serial
-// sums: planes of at most 64 positions with an LDS plan (33 images of 5 x 7 x 7 to 9 channels:
-// 11.9 against 13.4 us; 64 images of 16 x 20 x 20: 61 against 21 us), and layers under 2^22
-// products whose generic chunks have at most 64 positions (2 images of 61 x 7 x 7 to 43: 11.7
-// against 12.4 us; 3 images of 128 x 5 x 5 to 128, 2^23.2: 14.3 against 12.8 us).  Returns the
-// partial sums it leaves, 0 where it does not run.
+// on the matrix cores over groups of output rows (conv_weight_mfma.hip) where its estimated time is
+// under that of the kernel that would run in its place, in us:
+//   * the LDS kernel, 7 and 0.19 per position that a thread walks (fitted over 180 random layers):
+//     64 images of 16 x 20 x 20, 3 x 3: 61 against 21 us; 64 of 3 x 28 x 28 to 128, stride 2: 13.6
+//     against 16.1; never for planes of at most 64 (33 of 5 x 7 x 7 to 9: 11.9 against 13.4);
+//   * the generic one, 4.6 and the most of 0.11 per term of a thread's sum, its products at 1.15e-6
+//     (1e-6 in planes of at most 64) and its partial sums at 5e-6 (over 1070 layers): 2 of 61 x 7 x
+//     7 to 43, 3 x 3: 11.7 against 12.4; 77 of 576 x 19 x 19 to 1, whose tile is 31 rows of zeros:
+//     197 against 259; 52 of 127 x 8 x 8 to 156, 3 x 7 at stride 2, three positions an image: 48
+//     against 71; 32 of 64 x 56 x 56 to 64, 3 x 3: 5212 against 134.
+// Returns the partial sums it leaves, 0 where it does not run.
 uint32_t large_weight_partials(const ConvGeom &g) {
   if (g.groups != 1) return 0;
   const uint64_t oplane = static_cast<uint64_t>(g.oh) * g.ow;
-  if (weight_lds_plan(g).tile > 0) {
+  const LdsPlan lp = weight_lds_plan(g);
+  double other;
+  if (lp.tile > 0) {
     if (oplane <= 64) return 0;
+    other = 7 + 0.19 * lp.per_chunk * std::ceil(static_cast<double>(oplane) / lp.groups);
   } else {
     const uint64_t chunks = weight_chunks(g);
-    if (oplane * ((g.batch + chunks - 1) / chunks) <= 64 && products(g) < (1ull << 22)) return 0;
+    const uint64_t terms = oplane * ((g.batch + chunks - 1) / chunks);
+    if (terms <= 64 && products(g) < (1ull << 22)) return 0;  // short sums need no estimate
+    other = 4.6 + std::max({0.11 * terms, (oplane <= 64 ? 1e-6 : 1.15e-6) * products(g),
+                            5e-6 * chunks * weight_elems(g)});
   }
-  return oxh::conv_mfma::weight_partials(mfma_weight_dims(g));
+  const uint32_t partials = oxh::conv_mfma::weight_partials(mfma_weight_dims(g));
+  return partials > 0 && oxh::conv_mfma::weight_time(mfma_weight_dims(g)) < other ? partials : 0;
 }
 
 uint64_t weight_partial_bytes(const ConvGeom &g) {

@@ -53,6 +53,9 @@ struct WeightDims {
 // Partial sums it leaves, each of out_c * in_c * kh * kw values (1: the gradient itself); 0 when
 // the shape does not run here.
 uint32_t weight_partials(const WeightDims &d);
+// An estimate of its time in us, for a shape that runs here: the layout's cycles at 2.4 GHz, 1.8
+// times which, and 5 us, is what 1050 random layers took (within 1.4 times in nine of ten).
+double weight_time(const WeightDims &d);
 void weight_backward(hipStream_t s, const WeightDims &d, const float *gradient, const float *x,
                      float *out);
 

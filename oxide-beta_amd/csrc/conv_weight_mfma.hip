@@ -237,6 +237,7 @@ struct Plan {
   WeightArgs a{};
   int ct = 0;
   uint32_t chunks = 0, lds = 0;
+  double cycles = 0;  // estimated
 };
 
 Plan make_plan(const WeightDims &d) {
@@ -286,6 +287,7 @@ Plan make_plan(const WeightDims &d) {
     }
   }
   if (best.lds == 0) return best;
+  best.cycles = least;
   WeightArgs &a = best.a;
   a.C = d.in_c, a.M = d.out_c, a.H = d.h, a.W = d.w, a.OH = d.oh, a.OW = d.ow;
   a.KW = d.kw, a.taps = taps, a.stride = d.stride, a.pad = static_cast<int>(d.pad), a.wm = wm;
@@ -330,6 +332,8 @@ uint32_t weight_partials(const WeightDims &d) {
   const Plan &p = plan_of(d);
   return p.lds == 0 ? 0 : p.chunks * (4 / p.a.wm);
 }
+
+double weight_time(const WeightDims &d) { return 5.0 + 1.8 * plan_of(d).cycles / 2400; }
 
 void weight_backward(hipStream_t s, const WeightDims &d, const float *gradient, const float *x,
                      float *out) {

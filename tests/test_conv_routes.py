@@ -62,3 +62,20 @@ def test_input_gradient(case, serial):
 def test_pointwise(case, forward, backward):
     assert _serial(*case, 1, 1, 0, forward=True) == forward
     assert _serial(*case, 1, 1, 0, forward=False) == backward
+
+
+# batch, in, height, width, out, kernel, stride, padding
+@pytest.mark.parametrize("case,partials,bias", [
+    ((77, 576, 19, 19, 1, 3, 1, 1), 77, False),    # one output channel: a chunk per image
+    ((120, 220, 7, 7, 1, 3, 1, 0), 120, False),
+    ((62, 466, 6, 6, 3, 3, 2, 1), 62, False),
+    ((64, 3, 28, 28, 128, 3, 2, 1), 64, True),     # few columns: an image's sums in LDS
+    ((64, 1, 28, 28, 128, 3, 2, 1), 64, True),
+])
+def test_weight_gradient_of_few_rows_or_columns(case, partials, bias):
+    """The partial sums that the workspace holds are those of the kernels of one weight per thread
+    and of one image in LDS (with the bias sums)."""
+    n, cin, h, w, cout, k, s, pad = case
+    shape = ox.conv2d_shape(n, cin, h, w, cout, k, s, pad, 1)
+    sums = cout * cin * k * k + (cout if bias else 0)
+    assert ox.conv2d_workspace_size(shape) // (4 * sums) == partials
