@@ -1821,8 +1821,15 @@ oxh_status oxh::batch_norm_eval(hipStream_t stream, uint64_t batch, uint64_t cha
   const bool cross =
       quads && !vec && spatial > 4 && values < (1ull << 31) && tail != EvalTail::None;
   const uint64_t units = values / (vec || cross ? 4 : 1);
-  OXH_REQUIRE(units < (1ull << 31) - 2 * kMapBlock, OXH_INVALID_SHAPE,
-              std::string(name) + ": tensors are limited to 2^31 elements");
+  if (units >= (1ull << 31) - 2 * kMapBlock) {  // past the kernel's indexes: the launches it joins
+    st = oxh_batch_norm_running_inverse_std(stream, channels, epsilon, variance, inverse_std);
+    if (st != OXH_OK) return st;
+    st = oxh_batch_norm_apply(stream, batch, channels, spatial, input, weight, bias, mean,
+                              inverse_std, output);
+    if (st != OXH_OK || tail == EvalTail::None) return st;
+    return tail == EvalTail::Relu ? oxh_relu(stream, output, tail_output, values)
+                                  : oxh_add(stream, output, addend, tail_output, values);
+  }
   EvalArgs a{input, weight, bias, mean, variance, addend, inverse_std, output, tail_output,
              epsilon, static_cast<uint32_t>(units), static_cast<uint32_t>(channels),
              oxh::make_fastdiv(static_cast<uint32_t>(vec ? spatial / 4 : spatial)),

@@ -101,3 +101,40 @@ def test_planes_of_no_whole_units(dev, shape):
     for t, want in zip(nodes, one_by_one):
         assert np.isfinite(want).all()
         assert np.array_equal(program.value(t).host(), want), t
+
+
+class _Buffer:
+    """A program's buffer as torch takes it in."""
+
+    def __init__(self, view):
+        self.__cuda_array_interface__ = {"data": (view.ptr, False), "typestr": "<f4",
+                                         "shape": tuple(view.shape), "strides": None,
+                                         "version": 2}
+
+
+def test_tensors_past_32_bit_indexes(dev):
+    """2^31 values and more in planes of no whole float4: past the joined kernel's indexes, so its
+    launches one by one."""
+    shape = (1, 3, 26755, 26755)
+    x = tn.input(shape)
+    norm = _norm(3, np.random.default_rng(1))
+    a = norm(x)
+    b = a.relu()
+    program = tn.forward_program(b, [x])
+    xs, ys, zs = (torch.as_tensor(_Buffer(program.value(t)), device=dev).view(-1)
+                  for t in (x, a, b))
+    assert xs.numel() >= 1 << 31 and xs.numel() % 4 != 0
+    xs.normal_()
+    ys.fill_(float("nan"))
+    zs.fill_(float("nan"))
+    torch.cuda.synchronize()
+    program.run()
+    program.synchronize()
+    mean, variance = norm.state.running_mean, norm.state.running_variance
+    inverse = 1 / torch.sqrt(variance + 1e-5)
+    for start, c in ((0, 0), ((1 << 31) - (1 << 20), 2), (xs.numel() - (1 << 20), 2)):
+        v, y, z = (t[start:start + (1 << 20)] for t in (xs, ys, zs))
+        want = (v - mean[c]) * inverse[c] * norm.weight.data[c] + norm.bias.data[c]
+        assert torch.allclose(y, want, rtol=1e-6, atol=1e-6)  # a rounding in the square root
+        assert torch.equal(z, y.relu())
+    assert bool(zs.isfinite().all())
