@@ -1338,8 +1338,8 @@ oxh_status forward_train_impl(const char *name, oxh_stream stream, uint64_t batc
   OXH_REQUIRE(input && weight && bias && running_mean && running_variance && saved_mean &&
                   saved_inverse_std && output,
               OXH_INVALID_SHAPE, std::string(name) + ": null pointer");
-  st = check_workspace(name, make_geometry(batch, channels, spatial, false), workspace,
-                       workspace_bytes);
+  const Geometry g = make_geometry(batch, channels, spatial, false);
+  st = check_workspace(name, g, workspace, workspace_bytes);
   if (st != OXH_OK) return st;
   const uint64_t bytes = batch * channels * spatial * 4;
   st = no_overlap(name, output, bytes, {input}, bytes);
@@ -1348,6 +1348,9 @@ oxh_status forward_train_impl(const char *name, oxh_stream stream, uint64_t batc
                        momentum, epsilon};
   ChannelGeom cg = make_channel_geom(batch, channels, spatial);
   if (!use_channel(batch, channels, spatial)) {
+    // not written here, but refused as where planes of these sizes are reduced by slices
+    OXH_REQUIRE(!oxh::any_overlap(workspace, workspace_bytes_for(g), input, bytes),
+                OXH_INVALID_SHAPE, std::string(name) + ": workspace overlaps the input");
     const uint32_t units = static_cast<uint32_t>(wide_units(batch, spatial));
     cg.spatial_div = oxh::make_fastdiv((cg.spatial + 3) / 4);
     using W = decltype(&bn_wide_forward_kernel<1024, 2, true>);
@@ -1429,8 +1432,8 @@ oxh_status backward_train_impl(const char *name, oxh_stream stream, uint64_t bat
     const int size = wide_size(units);
     oxh::launch(wide[size][relu_out != nullptr], dim3(cg.channels),
                 dim3(size == 0 ? 256 : kWideThreads), 0, oxh::as_stream(stream), cg, units,
-                gradient, relu_out, input, weight, saved_mean, saved_inverse_std, input_gradient, weight_gradient,
-                bias_gradient, input_gradient_sum);
+                gradient, relu_out, input, weight, saved_mean, saved_inverse_std, input_gradient,
+                weight_gradient, bias_gradient, input_gradient_sum);
     return oxh::launched(name);
   }
   const int threads = channel_threads(cg);
