@@ -1201,11 +1201,23 @@ bool use_channel(uint64_t batch, uint64_t channels, uint64_t spatial) {
 // Whether the wide channel kernels take a shape the channel kernels do not: at most eight units
 // per thread, four where the channels are few (32 images of 32 x 28 x 28: 6.8 and 7.0 us forward
 // and ReLU backward by slices, 6.7 and 7.3 us by channels; 16 of 16 x 40 x 40, 6.7 against 7.2).
+// A forward over planes of whole units by slices has every CU load its share, which a channel's one
+// CU only matches up to about 6400 units below 80 channels and to nearly all 8192 below 128
+// (32 images of 64 x 32 x 32: 7.2 by slices, 8.5 us by channels; of 64 x 28 x 28: 7.6, 7.4; of 96 x
+// 32 x 32: 8.6, 9.2; of 128 x 32 x 32: 9.7, 9.9; 128 of 64 x 15 x 15, no whole units: 13.2, 8.2).
+// The backward stays by channels there: 7.3 by slices, 8.2 us for 64 x 32 x 32 without the input
+// gradient's channel sums, but with a ReLU behind 12.0 against 9.2 us.
 uint64_t wide_units(uint64_t batch, uint64_t spatial) { return batch * ((spatial + 3) / 4); }
 bool use_wide(uint64_t batch, uint64_t channels, uint64_t spatial) {
   return spatial >= kFlatSpatial && spatial >= 4 &&
          wide_units(batch, spatial) <= (channels < 64 ? kWideUnits / 2 : kWideUnits) &&
          batch * channels * spatial < (1ull << 31);
+}
+bool use_wide_forward(uint64_t batch, uint64_t channels, uint64_t spatial) {
+  const uint64_t most = spatial % 4 != 0 || channels >= 128 ? kWideUnits
+                        : channels < 80                     ? kWideUnits - kWideUnits * 7 / 32
+                                                            : kWideUnits - kWideUnits / 64;
+  return use_wide(batch, channels, spatial) && wide_units(batch, spatial) <= most;
 }
 
 ChannelGeom make_channel_geom(uint64_t batch, uint64_t channels, uint64_t spatial) {
@@ -1319,7 +1331,7 @@ oxh_status forward_train_impl(const char *name, oxh_stream stream, uint64_t batc
                               float *saved_mean, float *saved_inverse_std, float *output,
                               void *workspace, uint64_t workspace_bytes, bool relu,
                               const float *addend = nullptr) {
-  if (!use_channel(batch, channels, spatial) && !use_wide(batch, channels, spatial)) {
+  if (!use_channel(batch, channels, spatial) && !use_wide_forward(batch, channels, spatial)) {
     oxh_status st = launch_reduce_x(name, stream, batch, channels, spatial, input, workspace,
                                     workspace_bytes, nullptr);
     if (st != OXH_OK) return st;

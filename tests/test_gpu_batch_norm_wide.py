@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import oracle
+import oxide_hip as ox
 from helpers import (assert_within, check_batch_norm_backward, check_batch_norm_forward, host,
                      to_dev)
 
@@ -85,3 +86,30 @@ def test_training_step(module, dev, shape, lead):
         wide = got["dx"].astype(np.float64)
         assert_within(host(total), wide.sum((0, 2, 3)),
                       1e-6 * np.abs(wide).sum((0, 2, 3)) + 1e-7, "input gradient sums")
+
+
+@pytest.mark.parametrize("shape,by_slices", [
+    ((32, 64, 32, 32), True),     # few channels with many whole units: every CU loads a share
+    ((41, 79, 28, 28), True),
+    ((32, 96, 32, 32), True),
+    ((32, 64, 28, 24), False),    # up to six units per thread
+    ((41, 96, 28, 28), False),
+    ((32, 128, 32, 32), False),
+    ((26, 64, 35, 35), False),    # no whole units
+])
+def test_forward_of_few_channels(dev, shape, by_slices):
+    """The forward by slices leaves its partial sums in the workspace; the one by channels leaves
+    the workspace as it was."""
+    n, c, h, w = shape
+    x = torch.randn(shape, device=dev)
+    y = torch.empty_like(x)
+    one = [torch.ones(c, device=dev) for _ in range(6)]
+    size = ox.batch_norm_workspace_size(n, c, h * w)
+    work = torch.full((size // 4,), float("nan"), device=dev)
+    ox.check(ox.lib().oxh_batch_norm_forward_train(
+        ox.current_stream(), n, c, h * w, 0.1, 1e-5, x.data_ptr(), *(t.data_ptr() for t in one),
+        y.data_ptr(), work.data_ptr(), size))
+    assert bool(work.isnan().all()) != by_slices
+    ref = (x - x.mean((0, 2, 3), keepdim=True)) * (x.var((0, 2, 3), correction=0,
+                                                         keepdim=True) + 1e-5).rsqrt() + 1
+    assert float((y - ref).abs().max()) < 1e-4  # |x| < 7: some ulps of 2^-21
