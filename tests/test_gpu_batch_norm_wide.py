@@ -113,3 +113,48 @@ def test_forward_of_few_channels(dev, shape, by_slices):
     ref = (x - x.mean((0, 2, 3), keepdim=True)) * (x.var((0, 2, 3), correction=0,
                                                          keepdim=True) + 1e-5).rsqrt() + 1
     assert float((y - ref).abs().max()) < 1e-4  # |x| < 7: some ulps of 2^-21
+
+
+def test_values_that_are_not_finite(module, dev):
+    """An infinity or a NaN takes its own channel alone with it, in the forward and (there in the
+    incoming gradient) in the backward; the ReLU behind turns its NaN to 0."""
+    shape = (19, 72, 35, 35)
+    r = np.random.default_rng(3)
+    x, g = (r.standard_normal(shape).astype(np.float32) for _ in range(2))
+    gamma = r.uniform(0.5, 1.5, 72).astype(np.float32)
+    beta, rm, rv = np.full(72, 0.1, np.float32), np.zeros(72, np.float32), np.ones(72, np.float32)
+
+    def forward(values, relu):
+        call = module.batch_norm_relu_forward_train if relu else module.batch_norm_forward_train
+        out = [torch.empty(72, device=dev) for _ in range(2)] + [torch.empty(shape, device=dev)]
+        call(to_dev(values, dev), to_dev(gamma, dev), to_dev(beta, dev), to_dev(rm, dev),
+             to_dev(rv, dev), *out)
+        return [host(t) for t in out]
+
+    bad = x.copy()
+    bad[3, 5, 2, 7], bad[4, 6, 0, 1] = np.inf, np.nan
+    fine = np.delete(np.arange(72), [5, 6])
+    for relu in (False, True):
+        for a, b in zip(forward(x, relu), forward(bad, relu)):
+            assert np.array_equal(*(t[fine] if t.ndim == 1 else t[:, fine] for t in (a, b)))
+            if a.ndim > 1:
+                assert (b[:, 5:7] == 0).all() if relu else np.isnan(b[:, 5:7]).all()
+    ref = oracle.bn_forward(bad, gamma, beta, rm, rv, True, 0.1, 1e-5)[0]
+    assert np.array_equal(np.isnan(ref), np.isnan(forward(bad, False)[2]))
+
+    mean, inv, y = forward(x, True)
+    g[2, 9, 1, 1], g[1, 10, 3, 3], y[2, 9, 1, 1], y[1, 10, 3, 3] = np.nan, -np.inf, 1.0, 1.0
+    for relu in (False, True):
+        dx, dw, db = torch.empty(shape, device=dev), *(torch.empty(72, device=dev) for _ in "wb")
+        rest = (to_dev(x, dev), to_dev(gamma, dev), to_dev(mean, dev), to_dev(inv, dev), dx, dw, db)
+        if relu:
+            module.batch_norm_relu_backward_train(to_dev(g, dev), to_dev(y, dev), *rest)
+        else:
+            module.batch_norm_backward_train(to_dev(g, dev), *rest)
+        incoming = oracle.relu_backward(g, y) if relu else g
+        for got, want in zip((dx, dw, db), oracle.bn_backward(incoming, x, gamma, mean, inv, True)):
+            got = host(got)
+            assert np.array_equal(np.isnan(got), np.isnan(want))
+            assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+            np.testing.assert_allclose(got[np.isfinite(want)], want[np.isfinite(want)], rtol=1e-3,
+                                       atol=1e-3)

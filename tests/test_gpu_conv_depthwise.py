@@ -146,5 +146,4 @@ def test_small_layers_keep_their_pace(module, dev):
     times = [graph_time(lambda: module.conv2d_forward(shape, xd, wd, bd, y)),
              graph_time(lambda: module.conv2d_input_backward(shape, gd, wd, dx)),
              graph_time(lambda: module.conv2d_weight_backward(shape, gd, xd, dw))]
-    print(relu, times)
     assert sum(times) < 3 * 1.75 * relu, (relu, times)

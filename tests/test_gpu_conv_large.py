@@ -30,6 +30,10 @@ CASES = [
     (1, 24, 35, 33, 20, 1, 1, 1),     # a padded 1 x 1
     (20, 48, 17, 16, 66, 3, 1, 1),    # planes a per-image kernel holds, over 2^27 products
     (60, 64, 15, 14, 144, 3, 2, 1),
+    (12, 64, 3, 300, 64, 3, 1, 0),    # one output row a plane
+    (12, 61, 5, 300, 65, 3, 2, 0),    # two
+    (16, 24, 64, 63, 6, 3, 1, 1),     # six channels in a tile of 32
+    (16, 6, 64, 63, 24, 3, 1, 1),
 ]
 
 
@@ -102,6 +106,8 @@ WEIGHT_CASES = CASES + [
     (3, 64, 45, 44, 64, 3, 1, 1),
     (2, 18, 50, 47, 40, 7, 3, 2),
     (1, 2, 3, 300, 5, 3, 1, 1),
+    (40, 24, 3, 120, 33, 3, 1, 0),    # one output row, two
+    (40, 24, 4, 120, 33, 3, 1, 0),
     (4, 8, 18, 18, 32, 3, 1, 1),      # planes an LDS plan holds, over 64 positions
 ]
 

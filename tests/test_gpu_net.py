@@ -478,3 +478,73 @@ def test_whole_program_sums_more_convolutions_than_one_launch_takes():
     whole[0].replay()
     compare("replay")
     assert groups[0].steps() == whole[0].steps() == 2
+
+
+def test_step_over_larger_planes():
+    """Depthwise, 1 x 1 and 3 x 3 layers over planes of 121 to 441 values, each with its BatchNorm
+    and ReLU: every launch group of a step against the oracle, and whole runs and replays against
+    steps group by group, bit for bit.  BatchNorms of 64 and 72 channels form the bias gradient of
+    the convolution in front; depthwise and K x K weight gradients leave several partial sums for
+    the optimizer's launch.  A channel's sums have 14 112 terms: the oracle's running sums of more
+    than 2^14 would leave the 1e-5 * sum|terms| that the groups are held to."""
+    r = np.random.default_rng(67)
+    n, classes = 32, 10
+    layers = [(64, 64, 5, 2, 64), (64, 72, 1, 1, 1), (72, 72, 3, 1, 72), (72, 24, 3, 1, 1),
+              (24, 40, 3, 2, 1)]
+    xv = r.standard_normal((n, 64, 42, 42)).astype(np.float32)
+    targets = r.integers(0, classes, n).astype(np.float32)
+    values, size, several = [], 42, []
+    for cin, cout, k, s, groups in layers:
+        shape = ox.conv2d_shape(n, cin, size, size, cout, k, s, k // 2, groups)
+        several += [ox.conv2d_workspace_size(shape) >= 8 * cout * cin // groups * k * k]
+        size = ox.conv2d_output_size(shape)[0]
+        scale = np.float32((2 * groups / (cin * k * k)) ** 0.5)
+        values += [r.standard_normal((cout, cin // groups, k, k)).astype(np.float32) * scale,
+                   r.uniform(-0.1, 0.1, cout).astype(np.float32),
+                   r.uniform(0.5, 1.5, cout).astype(np.float32),
+                   r.uniform(-0.2, 0.2, cout).astype(np.float32)]
+    assert several == [True, True, False, True, True]
+    values += [r.standard_normal((classes, 40, 1, 1)).astype(np.float32) * np.float32(0.2),
+               r.uniform(-0.1, 0.1, classes).astype(np.float32)]
+
+    def build():
+        y = x = tn.input((n, 64, 42, 42))
+        t = tn.input((n,))
+        params = [nn.Parameter(v) for v in values]
+        q = [p.tensor() for p in params]
+        for i, (_, cout, k, s, groups) in enumerate(layers):
+            weight, bias, gamma, beta = q[4 * i:4 * i + 4]
+            y = y.conv2d(weight, bias, s, k // 2, groups)
+            y = y.batch_norm2d(gamma, beta, tn.BatchNormState(cout), True, 0.1, 1e-5).relu()
+        y = y.avg_pool2d((size, size), (size, size)).conv2d(q[-2], q[-1], 1, 0, 1)
+        loss = y.reshape((n, classes)).cross_entropy(t)
+        prog = tn.training_program(loss, nn.AdamW(1e-2, 1e-4))
+        prog.feed(x, xv)
+        prog.feed(t, targets)
+        return prog, loss, params
+
+    groups, whole = build(), build()
+
+    def compare(when):
+        torch.cuda.synchronize()
+        (pa, la, qa), (pb, lb, qb) = groups, whole
+        assert_bitexact(pb.value(lb).host(), pa.value(la).host(), f"{when}: loss")
+        for i, (u, v) in enumerate(zip(qa, qb)):
+            assert_bitexact(v.host(), u.host(), f"{when}: parameter {i}")
+            assert_bitexact(pb.gradient(v.tensor()).host(), pa.gradient(u.tensor()).host(),
+                            f"{when}: gradient {i}")
+
+    counts = _run_checked(groups[0])
+    assert counts["conv bias in batch norm backward"] >= 2
+    whole[0].run()
+    compare("run")
+    whole[0].capture()
+    for step in range(2):
+        for op in groups[0].ops:
+            op.launch()
+        whole[0].replay()
+        compare(f"replay {step}")
+    for op in groups[0].ops:
+        op.launch()
+    whole[0].run()
+    compare("run after replays")

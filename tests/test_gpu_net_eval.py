@@ -138,3 +138,44 @@ def test_tensors_past_32_bit_indexes(dev):
         assert torch.allclose(y, want, rtol=1e-6, atol=1e-6)  # a rounding in the square root
         assert torch.equal(z, y.relu())
     assert bool(zs.isfinite().all())
+
+
+@pytest.mark.parametrize("shape", [(3, 5, 6, 6), (2, 6, 7, 7), (1, 4, 3, 7), (64, 96, 7, 7),
+                                   (3, 5, 5, 7), (3, 5, 1, 1)])
+def test_inverse_deviations_and_values_that_are_not_finite(dev, shape):
+    """Infinities and NaN among the input and the running statistics, nothing, a ReLU (whose NaN is
+    0) and an addition behind: values and stored inverse deviations as the groups one by one leave
+    them, after a run and after replays with eager runs between."""
+    r = np.random.default_rng(sum(shape))
+    x = tn.input(shape)
+    norms = [_norm(shape[1], r) for _ in range(3)]
+    for norm, bad in zip(norms, (np.inf, np.nan, -2.0)):  # the last: a NaN square root
+        norm.state.running_variance[shape[1] - 2:shape[1] - 1] = bad
+    a = norms[0](x)
+    b = a.relu()
+    d = norms[1](b)
+    e = d.add(a)
+    f = norms[2](e)
+    program = tn.forward_program(f.mul(e), [x])
+    values = r.standard_normal(shape).astype(np.float32)
+    values.ravel()[1::19], values.ravel()[2::23], values.ravel()[3::29] = np.inf, np.nan, -np.inf
+    program.feed(x, values)
+    for op in program.ops:
+        op.launch()
+    program.synchronize()
+    groups = [op for op in program.ops if op.kind == "batch_norm2d_eval_forward"]
+    views = [program.value(t) for t in (a, b, d, e, f)] + [g.writes["inverse_std"] for g in groups]
+    assert len(views) == 8
+    want = [v.host() for v in views]
+    assert np.isnan(want[0]).any() and not np.isnan(want[1]).any()
+
+    def same(start):
+        for v in views:
+            v.copy_from(np.full(v.shape, 7.0, np.float32))
+        start()
+        program.synchronize()
+        return all(np.array_equal(v.host(), w, equal_nan=True) for v, w in zip(views, want))
+
+    assert same(program.run)
+    program.capture()
+    assert same(program.replay) and same(program.run) and same(program.replay)
