@@ -401,10 +401,11 @@ oxh_status oxh_adamw_multi_tensor_table_step(oxh_stream stream, float learning_r
  * input channels), and a pointwise input gradient with at least 256 output channels and fewer
  * than 512 32x32 tiles, sum four contiguous parts of the reduced channels and add the parts in
  * order; ungrouped 1x1, 3x3 and 5x5 layers over larger planes, or of over 2^27 products, sum on
- * the matrix cores.  Those sums, and the weight and bias gradients (fixed-order chunks), are
- * deterministic and within a few roundings (1e-5 * sum|terms|) of the serial sum; their products
- * are added by fused multiply-adds (one rounding per term), on the matrix cores (fp32 MFMA) for
- * the split tiles and the 32x32 weight-gradient tiles. */
+ * the matrix cores where that is the faster kernel (the two queries below tell).  Those sums, and
+ * the weight and bias gradients (fixed-order chunks), are deterministic and within a few roundings
+ * (1e-5 * sum|terms|) of the serial sum; their products are added by fused multiply-adds (one
+ * rounding per term), on the matrix cores (fp32 MFMA) for the split tiles, the 32x32
+ * weight-gradient tiles, the large 1x1 and KxK layers and ungrouped KxK weight gradients. */
 typedef struct oxh_conv2d_shape {
   uint64_t batch, in_channels, height, width;
   uint64_t out_channels, kernel_h, kernel_w;
@@ -416,8 +417,8 @@ typedef struct oxh_conv2d_shape {
 int oxh_conv2d_forward_serial(const oxh_conv2d_shape *shape);
 /* The same for the input gradient (oxh_conv2d_input_backward, _accumulate and the input
  * gradient of oxh_conv2d_backward): 0 when it sums four ordered parts over the output channels
- * (pointwise) or on the matrix cores (stride-2 K x K, large layers).  No counterpart in the reference (its CPU
- * path has one order). */
+ * (pointwise) or on the matrix cores (stride-2 K x K, large layers).  No counterpart in the
+ * reference (its CPU path has one order). */
 int oxh_conv2d_input_backward_serial(const oxh_conv2d_shape *shape);
 oxh_status oxh_conv2d_output_size(const oxh_conv2d_shape *shape, uint64_t *out_h,
                                   uint64_t *out_w);

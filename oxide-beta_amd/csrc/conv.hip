@@ -1442,10 +1442,10 @@ __global__ __launch_bounds__(256) void conv2d_bias_kernel(BiasArgs a) { bias_blo
 // More than kWideBias terms per channel: a block of 1024 threads per channel, eight 128-bit loads
 // in flight per thread (scalar ones where planes are not whole float4s), fixed-order wave sums
 // added in wave order.  One wave per channel ran at the latency of its four loads in flight: 32
-// images of 64 x 56 x 56 took 131 us and now 8 us; 32 of 32 x 112 x 112, 547 us and now 22 us (32
-// blocks: bound by what one CU loads).  A channel's terms have to meet in one block, as the entry
-// point has no workspace.  The line is where a wave's dependent rounds of loads (6272 terms: 13 us
-// on the device) outlast the block's barrier and sums (4 us).
+// images of 64 x 56 x 56 took 125 us and now 6.5 us; 32 of 32 x 112 x 112, 550 us and now 20 us (32
+// blocks: bound by what one CU loads).  A channel's terms have to meet in one block: callers of the
+// bias entry point may pass no workspace.  The line is where a wave's dependent rounds of loads
+// (6272 terms: 13 us on the device) outlast the block's barrier and sums (4 us).
 constexpr uint32_t kWideBias = 4096, kPairedBias = 7168;
 constexpr int kWideBiasThreads = 1024;
 template <bool Vec>
@@ -2922,9 +2922,9 @@ bool large_pointwise(const ConvGeom &g, bool forward) {
 }
 
 // The bias kernel of a layer.  A 1 x 1 backward in one launch sums the bias in passing, a wave per
-// channel, which outlasts its products only from about 7000 terms on (42 images of 30 x 10 x 10 to 9,
-// 4200 terms: 7.6 us, 10.2 with a launch of its own; 12 000 terms: 0.77 of the time); the bias entry
-// point follows, so that both leave the same bits.
+// channel, which outlasts its products only from about 7000 terms on (42 images of 30 x 10 x 10 to
+// 9, 4200 terms: 7.6 us, 10.2 with a launch of its own; 12 000 terms: 0.77 of the time); the bias
+// entry point follows, so that both leave the same bits.
 bool wide_bias(const ConvGeom &g) {
   const bool paired = pointwise(g) && !large_pointwise(g, false);
   return static_cast<uint64_t>(g.batch) * g.oh * g.ow > (paired ? kPairedBias : kWideBias);
@@ -2997,12 +2997,12 @@ bool depthwise_single_pass(const ConvGeom &g) {
 }
 
 // Those of them with four and more columns run in tiles (conv_depthwise.hip) from five million
-// products on, 2.8 million in a stride-2 forward: a tile's rows of loads and sums follow each other,
-// 4 to 6 us, which small layers do not hide (2 images of 39 x 10 x 10, 3 x 3: 2.5 against 4.4 us
-// forward and input gradient; at the line both take 4 to 5 us; 64 of 192 x 28 x 28, 5 x 5: 124
-// against 21).  One channel is also an ungrouped layer, whose kernels take as long a chain: tiles
-// from 196 outputs on, and for every input gradient (8 images of 1 x 86 x 86, 5 x 5, stride 2: 174
-// against 4 us).
+// products on, 2.8 million in a stride-2 forward: a tile's rows of loads and sums follow each
+// other, 4 to 6 us, which small layers do not hide (2 images of 39 x 10 x 10, 3 x 3: 2.5 against
+// 4.4 us forward and input gradient; at the line both take 4 to 5 us; 64 of 192 x 28 x 28, 5 x 5:
+// 124 against 21).  One channel is also an ungrouped layer, whose kernels take as long a chain:
+// tiles from 196 outputs on, and for every input gradient (8 images of 1 x 86 x 86, 5 x 5, stride
+// 2: 174 against 4 us).
 bool tiled_depthwise(const ConvGeom &g, bool forward) {
   if (!depthwise_single_pass(g) || !oxh::conv_mfma::takes_depthwise(mfma_dims(g))) return false;
   if (g.in_c == 1 && (!forward || g.oh * g.ow > 196)) return true;
@@ -3010,13 +3010,13 @@ bool tiled_depthwise(const ConvGeom &g, bool forward) {
                           (forward ? g.oh * g.ow : g.h * g.w);
   return values * g.kh * g.kw >= (forward && g.stride == 2 ? 2800000u : 5000000u);
 }
-// Their weight gradient, by the outputs of a channel, which one block or a few walk: 3 x 3 from 4000
-// on (stride 2: 2900), 5 x 5 from 2080 (stride 2: 1040), or 1000 where 128 channels and more fill
-// the chip (19 images of 3 x 23 x 23, 3 x 3, stride 2: 3.0 against 4.1 us; 2 of 58 x 50 x 50: 6.2
-// against 6.5; 17 of 293 x 14 x 15, 5 x 5: 15 against 8).  A 3 x 3 kernel at stride 2 keeps a thread
-// per position up to 64 of a plane, where half of each tile's loads would be for nothing (32 images
-// of 576 x 14 x 14: 10.1 against 13.4 us; 96 x 56 x 56: 39 against 21 us), and up to eight columns
-// where the channels fill the chip without chunks (98 of 469 x 99 x 11: 75 against 113 us).
+// Their weight gradient, by the outputs of a channel, which one block or a few walk: 3 x 3 from
+// 4000 on (stride 2: 2900), 5 x 5 from 2080 (stride 2: 1040), or 1000 where 128 channels and more
+// fill the chip (19 images of 3 x 23 x 23, 3 x 3, stride 2: 3.0 against 4.1 us; 2 of 58 x 50 x 50:
+// 6.2 against 6.5; 17 of 293 x 14 x 15, 5 x 5: 15 against 8).  A 3 x 3 kernel at stride 2 keeps a
+// thread per position up to 64 of a plane, where half of each tile's loads would be for nothing (32
+// images of 576 x 14 x 14: 10.1 against 13.4 us; 96 x 56 x 56: 39 against 21 us), and up to eight
+// columns where the channels fill the chip without chunks (98 of 469 x 99 x 11: 75 against 113 us).
 bool tiled_depthwise_weight(const ConvGeom &g) {
   if (!depthwise_single_pass(g) || !oxh::conv_mfma::takes_depthwise(mfma_dims(g))) return false;
   const bool strided = g.stride == 2;

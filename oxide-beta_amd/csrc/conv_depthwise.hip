@@ -6,7 +6,8 @@
 // loads stop repeating: a thread per output reads its K * K inputs one by one.  Here a thread takes
 // a tile of outputs and reads each row of inputs under it once, four values per load at any
 // alignment.  64 images of 192 x 28 x 28, 5 x 5: forward 124 -> 21 us, input gradient 140 -> 21 us
-// (the tensors alone: 15 us); 32 of 32 x 112 x 112, 3 x 3: 44 -> 19 and 76 -> 19 us (20 us).
+// (both tensors once, at the 6.24 TB/s of a large copy: 12.4 us); 32 of 32 x 112 x 112, 3 x 3:
+// 44 -> 19 and 76 -> 19 us (16.5 us).
 // Sums keep the CPU path's order (bias, then taps by row and column; the input gradient by output
 // row and column), one multiplication and one addition per tap: bit-identical.  An input outside
 // the plane is a +0 operand in place of a skipped tap: the same sum while the weights are finite
@@ -230,9 +231,10 @@ __global__ __launch_bounds__(256, 4) void depthwise_input_s2_kernel(DepthArgs a,
 // outputs, whose products go to one sum per tap by fused multiply-adds; wave sums in a fixed order,
 // waves in order.  Operands outside are +0; a thread that ends with a sum that is not finite walks
 // its items again, skipping them.  Bound by the loads a CU issues: the tile shares each row of
-// inputs among its outputs' rows.  64 images of 192 x 28 x 28, 5 x 5: 157 -> 29 us; 32 of 64 x 28 x 28, 5 x 5:
-// 51 -> 14.5 us; 32 of 32 x 112 x 112, 3 x 3: 305 -> 29 us.  5 x 5 kernels are bound to three waves
-// per SIMD (bound to four, their rows spilled: 14 against 18 us for 192 x 28 x 28 at stride 2).
+// inputs among its outputs' rows.  64 images of 192 x 28 x 28, 5 x 5: 157 -> 29 us; 32 of 64 x 28 x
+// 28, 5 x 5: 51 -> 14.5 us; 32 of 32 x 112 x 112, 3 x 3: 305 -> 29 us.  5 x 5 kernels are bound to
+// three waves per SIMD (bound to four, their rows spilled: 14 against 18 us for 192 x 28 x 28 at
+// stride 2).
 struct DepthWeightArgs {
   const float *g, *x;
   float *dw;
